@@ -66,15 +66,14 @@ enum sfg_dtype { SFG_F32 = 0, SFG_BF16 = 1, SFG_I8 = 2, SFG_I32 = 3 /* taps only
 enum sfg_layout { SFG_LAYOUT_NK = 0, SFG_LAYOUT_TILED = 1 };
 
 /* Output tile of the bf16 direct-to-LDS GEMM family that runs the prefill
- * projections and grouped expert GEMMs (bf16 weights, >= 1024 rows, k % 32 == 0).
+ * projections and grouped expert GEMMs (bf16 weights, >= 1024 rows, k % 64 == 0).
  * A plan policy, not a numeric choice: every tile gives bit-identical results
  * (each output is one fp32 accumulation in k order).  Ignored by the other GEMM
  * paths (skinny decode GEMV, fp32, int8 and small-M kernels).  The plan
  * optimiser (ExecutablePlanOptimizer, decoder_compiler.cpp:750-861) searches it. */
 enum sfg_gemm_tile {
-    SFG_TILE_AUTO = 0,       /* the largest tile that still gives >= 512 workgroups
-                                (256 x 256 as V); grouped products take V from 128
-                                workgroups up                                       */
+    SFG_TILE_AUTO = 0,       /* the fastest by estimate: 256 x 256 as V, or a smaller
+                                tile where that leaves compute units idle          */
     SFG_TILE_256x256_PP = 1, /* eight waves as two ping-pong groups of four          */
     SFG_TILE_256x256_W8 = 2, /* eight waves (2 x 4), 128 x 64 per wave               */
     SFG_TILE_256x256_W4 = 3, /* four waves (2 x 2), 128 x 128 per wave               */
@@ -170,11 +169,12 @@ int sfg_hip_rmsnorm_v1(const float* x, const float* w, void* y, int y_dtype, int
  * SFG_ERR_UNSUPPORTED.
  * c_dtype: SFG_F32 or SFG_BF16.  Replaces execute(LoopIR) (runtime.cpp:581-626)
  * for the four projections and quantized_invoke (next_milestones.cpp:50-69).
- * workspace: sfg_hip_gemm_workspace_v1 bytes.  Non-zero only for 33..64 dense
- * rows with k a multiple of 512 (>= 1024) and N (2N for GLU) a multiple of
- * 128: those run split-K over 512-k slices with fp32 partial sums in the
- * workspace, summed in slice order.  With a smaller workspace (or NULL) the
- * same shapes run the single-pass decode kernel instead.
+ * workspace: sfg_hip_gemm_workspace_v1 bytes, holding the fp32 partial sums of
+ * split-K products, which are summed in split order.  Non-zero for 33..64 dense
+ * rows with k a multiple of 512 (>= 1024) and N (2N for GLU) a multiple of 128,
+ * and for 65..1023 dense rows whose tiles alone leave compute units idle (at
+ * most 64 MiB).  With a smaller workspace (or NULL) the same products run with
+ * fewer splits or in a single pass.
  * b_layout SFG_LAYOUT_TILED is read by the decode GEMV only: bf16 / int8 B,
  * at most 64 rows (grouped: 512 in all), K % 128 == 0 and N % 16 == 0;
  * other shapes with tiled B return SFG_ERR_UNSUPPORTED. */

@@ -362,7 +362,8 @@ int sfg_hip_rmsnorm_v1(const float* x, const float* w, void* y, int y_dtype, int
 }
 
 size_t sfg_hip_gemm_workspace_v1(int64_t m, int64_t n, int64_t k) {
-    return sfg::gemm_workspace_bytes(m, 2 * n, k);
+    const size_t plain = sfg::gemm_workspace_bytes(m, n, k), glu = sfg::gemm_workspace_bytes(m, 2 * n, k);
+    return plain > glu ? plain : glu;
 }
 
 int sfg_hip_gemm_v1(const sfg_gemm_args* a, void* workspace, size_t workspace_bytes, void* stream) {

@@ -1,0 +1,425 @@
+// sfg_gemm_ring.hip -- the MFMA GEMM of the middle sizes (65 rows up): bf16 or
+// int8 weights, dense or grouped, optionally split over K.
+#include "sfg_gemm_tile.hpp"
+
+namespace sfg {
+
+// ===========================================================================
+// Ring GEMM: BM x BN output tile, four waves in a 2 x 2 grid, K in slabs of 64
+// through a ring of NS LDS stages filled by DMA (global -> LDS, no registers).
+//
+// With 65 .. ~1000 rows a launch has one or two tiles per CU, so nothing else
+// on the CU hides a slab's latency: what bounds the tile is how many bytes it
+// keeps in flight.  The ring holds most of the CU's 160 KB for one workgroup
+// (NS - 1 slabs of 16 - 32 KB in flight), one barrier per 64 k.
+//
+// A rows are 128 B with 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7);
+// bf16 B rows the same; int8 B rows are 64 B with chunk c in slot
+// c ^ ((r >> 2) & 3), converted to bf16 (exactly) between the LDS read and the
+// MFMA, under the matrix pipe.  The MFMA k order is free as long as A and B
+// agree: int8 step j of a slab takes k = 32 (j / 2) + 16 half + 8 (j % 2) + [0, 8),
+// so one 16-byte read feeds two steps.
+// A K that is an odd multiple of 32 ends in half a slab: its upper chunks are
+// loaded from past the end of the buffer resource, which returns zeros.
+//
+// SPLIT: blockIdx.y takes a contiguous range of slabs and the fp32 sums go to
+// part [split][m][B rows]; gemm_splitk_reduce_kernel adds them in split order.
+// ===========================================================================
+template <int BDT, int BM, int BN>
+constexpr int kRingStageElems = BM * 64 + BN * (BDT == SFG_I8 ? 32 : 64);  // uint16 units
+
+template <int BDT, int BM, int BN, int NW, int NS, int EPI, bool SPLIT>
+__global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int tiles_m, int tiles_n, float* part) {
+    constexpr bool kGlu = EpiTraits<EPI>::glu;
+    constexpr bool kI8 = BDT == SFG_I8;
+    constexpr int kWavesM = NW / 2;
+    constexpr int WM = BM / (32 * kWavesM), WN = BN / 64;  // 32 x 32 tiles per wave
+    constexpr int kStage = kRingStageElems<BDT, BM, BN>;
+    constexpr int kBRow = kI8 ? 32 : 64;                 // uint16 units per B row in LDS
+    constexpr int kLoadsA = BM / (8 * NW), kLoadsB = BN / ((kI8 ? 16 : 8) * NW);  // DMA instructions per wave per slab
+    constexpr int kLoads = kLoadsA + kLoadsB;
+    static_assert(NS >= 3 && NS <= 6 && (NS - 2) * kLoads < 64, "ring depth");
+    static_assert(!kGlu || WN % 2 == 0, "GLU tiles pair gate and up blocks");
+    // one array per stage: the compiler tells loads in flight from the stage
+    // being read by the array
+    __shared__ __attribute__((aligned(1024))) uint16_t s0[kStage];
+    __shared__ __attribute__((aligned(1024))) uint16_t s1[kStage];
+    __shared__ __attribute__((aligned(1024))) uint16_t s2[kStage];
+    __shared__ __attribute__((aligned(1024))) uint16_t s3[NS > 3 ? kStage : 8];
+    __shared__ __attribute__((aligned(1024))) uint16_t s4[NS > 4 ? kStage : 8];
+    __shared__ __attribute__((aligned(1024))) uint16_t s5[NS > 5 ? kStage : 8];
+
+    const int tid = threadIdx.x;
+    const int lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave >> 1, wn = wave & 1;
+    constexpr int kOutCols = kGlu ? BN / 2 : BN;
+
+    int g;
+    int64_t rb, re, tm, tn;
+    if (!dma_tile_coords<BM>(p, tiles_m, tiles_n, g, rb, re, tm, tn)) return;
+    const int64_t row0 = rb + tm * BM;
+    if (row0 >= re) return;
+    const int64_t ncol0 = tn * kOutCols;
+    const float* scales = p.scales ? p.scales + static_cast<int64_t>(g) * p.s_group_stride : nullptr;
+
+    // slabs of this workgroup
+    const int64_t all_slabs = (p.k + 63) / 64;
+    int64_t slab0 = 0, slab1 = all_slabs;
+    if constexpr (SPLIT) {
+        slab0 = all_slabs * blockIdx.y / gridDim.y;
+        slab1 = all_slabs * (blockIdx.y + 1) / gridDim.y;
+    }
+    const bool half_tail = p.k % 64 != 0;  // the last slab holds 32 k
+
+    // DMA sources.  A: instruction i fills rows 8 (4 i + wave) + lane / 8, slot
+    // lane % 8.  Rows past the tile read its first row (never stored); a
+    // gathered id outside A starts past A's resource and reads zeros.
+    const uint32_t a_bytes = static_cast<uint32_t>(p.a_rows_limit * p.lda * 2);
+    const buf_rsrc ra = make_rsrc(p.a, a_bytes);
+    uint32_t a_off[kLoadsA];
+    const int a_row = lane >> 3, a_slot = lane & 7;
+#pragma unroll
+    for (int i = 0; i < kLoadsA; ++i) {
+        const int local = (NW * i + wave) * 8 + a_row;
+        const int64_t r = row0 + local;
+        int64_t src = r < re ? r : row0;
+        if (p.a_rows) src = p.a_rows[src];
+        const int chunk = a_slot ^ ((local >> 1) & 7);
+        a_off[i] = (src < 0 || src >= p.a_rows_limit) ? a_bytes
+                                                      : static_cast<uint32_t>((src * p.lda + chunk * 8) * 2);
+    }
+    constexpr int kBElem = kI8 ? 1 : 2;
+    const uint32_t b_bytes = static_cast<uint32_t>((kGlu ? 2 : 1) * p.n * p.ldb * kBElem);
+    const buf_rsrc rbs = make_rsrc(static_cast<const char*>(p.b) + static_cast<int64_t>(g) * p.b_group_stride * kBElem,
+                                   b_bytes);
+    uint32_t b_off[kLoadsB];
+#pragma unroll
+    for (int i = 0; i < kLoadsB; ++i) {
+        const int local = kI8 ? (NW * i + wave) * 16 + (lane >> 2) : (NW * i + wave) * 8 + (lane >> 3);
+        const int chunk = kI8 ? (lane & 3) ^ ((local >> 2) & 3) : (lane & 7) ^ ((local >> 1) & 7);
+        int64_t brow;
+        if (kGlu) {
+            const int block = local >> 5;
+            const int64_t col = ncol0 + (block >> 1) * 32 + (local & 31);
+            brow = col < p.n ? ((block & 1) ? p.n + col : col) : 0;
+        } else {
+            const int64_t col = ncol0 + local;
+            brow = col < p.n ? col : 0;
+        }
+        b_off[i] = static_cast<uint32_t>((brow * p.ldb) * kBElem + chunk * 16);
+    }
+    // DMA instructions [i0, i1) of slab s into stage st (A's first, then B's).
+    // Slabs past the end re-fetch the last one.
+    auto issue = [&](uint16_t* st, int64_t s, int i0, int i1) __attribute__((always_inline)) {
+        const int64_t sl = min(s, slab1 - 1);
+        const bool tail = half_tail && sl == all_slabs - 1;  // wave-uniform
+        const uint32_t ka = static_cast<uint32_t>(sl * 128), kb = static_cast<uint32_t>(sl * 64 * kBElem);
+#pragma unroll
+        for (int i = 0; i < kLoadsA; ++i) {
+            if (i < i0 || i >= i1) continue;
+            const int local = (NW * i + wave) * 8 + a_row;
+            const uint32_t off = tail && (a_slot ^ ((local >> 1) & 7)) >= 4 ? a_bytes : a_off[i];
+            lds_dma16_buf(ra, off, ka, st + (NW * i + wave) * 8 * 64);
+        }
+#pragma unroll
+        for (int i = 0; i < kLoadsB; ++i) {
+            if (i + kLoadsA < i0 || i + kLoadsA >= i1) continue;
+            const int local = kI8 ? (NW * i + wave) * 16 + (lane >> 2) : (NW * i + wave) * 8 + (lane >> 3);
+            const bool up = kI8 ? ((lane & 3) ^ ((local >> 2) & 3)) >= 2 : ((lane & 7) ^ ((local >> 1) & 7)) >= 4;
+            const uint32_t off = tail && up ? b_bytes : b_off[i];
+            lds_dma16_buf(rbs, off, kb, st + BM * 64 + (NW * i + wave) * (kI8 ? 16 : 8) * kBRow);
+        }
+    };
+
+    floatx16 acc[WM][WN];
+#pragma unroll
+    for (int i = 0; i < WM; ++i)
+#pragma unroll
+        for (int j = 0; j < WN; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) acc[i][j][r] = 0.f;
+
+    const int l32 = lane & 31, khalf = lane >> 5;
+    const int asw = (l32 >> 1) & 7, bsw = kI8 ? (l32 >> 2) & 3 : asw;
+    // A and B fragments of 16-k step J (int8: raw, both steps of the 32-k group
+    // at even J)
+    bf16x8 fa[2][WM], fb[2][kI8 ? 1 : WN];
+    uint4 fq[2][kI8 ? WN : 1];
+    auto frags = [&](const uint16_t* st, auto j_c) __attribute__((always_inline)) {
+        constexpr int J = decltype(j_c)::value;
+        const int ca = kI8 ? 4 * (J >> 1) + 2 * khalf + (J & 1) : 2 * J + khalf;
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+            fa[J & 1][i] = as_bf16x8(*reinterpret_cast<const uint4*>(
+                st + (wm * (BM / kWavesM) + i * 32 + l32) * 64 + (ca ^ asw) * 8));
+        const uint16_t* sb = st + BM * 64;
+        if constexpr (kI8) {
+            if constexpr ((J & 1) == 0) {
+#pragma unroll
+                for (int i = 0; i < WN; ++i)
+                    fq[(J >> 1) & 1][i] = *reinterpret_cast<const uint4*>(
+                        sb + (wn * (BN / 2) + i * 32 + l32) * kBRow + (((J & 2) + khalf) ^ bsw) * 8);
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < WN; ++i)
+                fb[J & 1][i] = as_bf16x8(*reinterpret_cast<const uint4*>(
+                    sb + (wn * (BN / 2) + i * 32 + l32) * kBRow + ((2 * J + khalf) ^ bsw) * 8));
+        }
+    };
+    auto mfmas = [&](auto j_c) __attribute__((always_inline)) {
+        constexpr int J = decltype(j_c)::value;
+        bf16x8 b[WN];
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+            if constexpr (kI8) {
+                const uint4 q = fq[(J >> 1) & 1][j];
+                b[j] = (J & 1) ? as_bf16x8(i8x8_to_bf16x8(q.z, q.w)) : as_bf16x8(i8x8_to_bf16x8(q.x, q.y));
+            } else {
+                b[j] = fb[J & 1][j];
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int j = 0; j < WN; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fa[J & 1][i], b[j], acc[i][j], 0, 0, 0);
+    };
+    using J0 = std::integral_constant<int, 0>;
+    using J1 = std::integral_constant<int, 1>;
+    using J2 = std::integral_constant<int, 2>;
+    using J3 = std::integral_constant<int, 3>;
+    // One slab: each step's fragments are read under the step before it.  The
+    // barrier that publishes slab s + 1 also retires every read of slab s, so
+    // the next slab's DMA may overwrite that stage.  Every slab issues the same
+    // number of loads (past the end it re-fetches the last one), so the wait is
+    // always for all but the newest NS - 2 groups.
+    auto slab = [&](int64_t s, const uint16_t* cur, uint16_t* prev, const uint16_t* next) __attribute__((always_inline)) {
+        constexpr int kM = WM * WN, kR = WM + WN, kL1 = (kLoads + 2) / 3, kL2 = (2 * kLoads + 2) / 3;
+        frags(cur, J1{});
+        issue(prev, s + NS - 1, 0, kL1);
+        mfmas(J0{});
+        spread_reads_loads<kM, kR, kL1>();
+        __builtin_amdgcn_sched_barrier(0);
+        frags(cur, J2{});
+        issue(prev, s + NS - 1, kL1, kL2);
+        mfmas(J1{});
+        spread_reads_loads<kM, kR, kL2 - kL1>();
+        __builtin_amdgcn_sched_barrier(0);
+        frags(cur, J3{});
+        issue(prev, s + NS - 1, kL2, kLoads);
+        mfmas(J2{});
+        spread_reads_loads<kM, kR, kLoads - kL2>();
+        __builtin_amdgcn_sched_barrier(0);
+        wait_vmem_lds<(NS - 2) * kLoads>();
+        barrier_no_fence();
+        frags(next, J0{});
+        mfmas(J3{});
+        spread_reads_loads<kM, kR, 0>();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    issue(s0, slab0, 0, kLoads);
+    issue(s1, slab0 + 1, 0, kLoads);
+    if constexpr (NS > 3) issue(s2, slab0 + 2, 0, kLoads);
+    if constexpr (NS > 4) issue(s3, slab0 + 3, 0, kLoads);
+    if constexpr (NS > 5) issue(s4, slab0 + 4, 0, kLoads);
+    wait_vmem_lds<(NS - 2) * kLoads>();
+    barrier_no_fence();
+    frags(s0, J0{});
+    int64_t s = slab0;
+    if constexpr (NS == 3) {
+        for (; s + 3 <= slab1; s += 3) {
+            slab(s, s0, s2, s1);
+            slab(s + 1, s1, s0, s2);
+            slab(s + 2, s2, s1, s0);
+        }
+        if (s < slab1) slab(s, s0, s2, s1);
+        if (s + 1 < slab1) slab(s + 1, s1, s0, s2);
+    } else if constexpr (NS == 4) {
+        for (; s + 4 <= slab1; s += 4) {
+            slab(s, s0, s3, s1);
+            slab(s + 1, s1, s0, s2);
+            slab(s + 2, s2, s1, s3);
+            slab(s + 3, s3, s2, s0);
+        }
+        if (s < slab1) slab(s, s0, s3, s1);
+        if (s + 1 < slab1) slab(s + 1, s1, s0, s2);
+        if (s + 2 < slab1) slab(s + 2, s2, s1, s3);
+    } else if constexpr (NS == 5) {
+        for (; s + 5 <= slab1; s += 5) {
+            slab(s, s0, s4, s1);
+            slab(s + 1, s1, s0, s2);
+            slab(s + 2, s2, s1, s3);
+            slab(s + 3, s3, s2, s4);
+            slab(s + 4, s4, s3, s0);
+        }
+        if (s < slab1) slab(s, s0, s4, s1);
+        if (s + 1 < slab1) slab(s + 1, s1, s0, s2);
+        if (s + 2 < slab1) slab(s + 2, s2, s1, s3);
+        if (s + 3 < slab1) slab(s + 3, s3, s2, s4);
+    } else {
+        for (; s + 6 <= slab1; s += 6) {
+            slab(s, s0, s5, s1);
+            slab(s + 1, s1, s0, s2);
+            slab(s + 2, s2, s1, s3);
+            slab(s + 3, s3, s2, s4);
+            slab(s + 4, s4, s3, s5);
+            slab(s + 5, s5, s4, s0);
+        }
+        if (s < slab1) slab(s, s0, s5, s1);
+        if (s + 1 < slab1) slab(s + 1, s1, s0, s2);
+        if (s + 2 < slab1) slab(s + 2, s2, s1, s3);
+        if (s + 3 < slab1) slab(s + 3, s3, s2, s4);
+        if (s + 4 < slab1) slab(s + 4, s4, s3, s5);
+    }
+    wait_vmem<0>();
+
+    if constexpr (SPLIT) {
+        // fp32 sums of this slab range, B row order
+        const int64_t nb = (kGlu ? 2 : 1) * p.n;
+        float* const out = part + static_cast<int64_t>(blockIdx.y) * p.m * nb;
+#pragma unroll
+        for (int i = 0; i < WM; ++i)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int64_t row = row0 + wm * (BM / kWavesM) + i * 32 + 8 * (r >> 2) + 4 * khalf + (r & 3);
+                if (row >= re) continue;
+#pragma unroll
+                for (int j = 0; j < WN; ++j) {
+                    const int block = wn * WN + j;
+                    const int64_t col = kGlu ? ncol0 + (block >> 1) * 32 + l32 : ncol0 + block * 32 + l32;
+                    if (col < p.n) out[row * nb + (kGlu && (block & 1) ? p.n + col : col)] = acc[i][j][r];
+                }
+            }
+    } else {
+        // 8 KB of staging per wave
+        constexpr int kPer = kStage / 4096;  // waves' regions per stage array
+        static_assert(EPI != kEpiQkvRope || WM != WN || WM == 1 || NW <= 3 * kPer, "staging fits three stage arrays");
+        float* const qkv_stage = reinterpret_cast<float*>((wave < kPer ? s0 : wave < 2 * kPer ? s1 : s2) + (wave % kPer) * 4096);
+        dma_tile_epilogue<BM, BN, NW, EPI, false, kWavesM>(p, acc, wm, wn, row0, ncol0, re, scales, qkv_stage);
+    }
+}
+
+// ===========================================================================
+// Host side: tile and split choice.
+// ===========================================================================
+namespace {
+
+// One tile of the choice: its workgroups per CU and microseconds per 64-k slab
+// with every CU busy (bf16 / int8 weights).  The slab times are what the L2
+// miss path gives one CU: it moves 45 - 55 KB/us whatever the ring depth (four
+// and five stages, and 32 to 256 workgroups, measured within 3%), so a slab
+// costs its bytes, and larger tiles win until they leave CUs idle.
+struct RingTile {
+    int tile, bm, bn, per_cu;
+    float us_bf16, us_i8;
+    bool glu;
+};
+constexpr RingTile kRingTiles[] = {
+    {kRingTileV, 256, 256, 1, 1.40f, 0.f, true},
+    {kRingTile256x128, 256, 128, 1, 1.10f, 0.90f, true},
+    {kRingTile128x128, 128, 128, 1, 0.67f, 0.54f, true},
+    {kRingTile128x64, 128, 64, 1, 0.45f, 0.42f, false},
+    {kRingTile64x64, 64, 64, 2, 0.53f, 0.45f, false},
+};
+constexpr int kRingCus = 256;
+constexpr size_t kRingMaxPart = size_t(64) << 20;  // bytes of split-K partials
+
+}  // namespace
+
+RingPlan ring_plan(int b_dtype, int64_t m, int64_t n, int64_t k, bool glu, int groups, bool may_split,
+                   bool allow_v, size_t workspace) {
+    const int64_t slabs = (k + 63) / 64;
+    const int64_t nb = glu ? 2 * n : n;
+    RingPlan best{};
+    float best_us = 0.f;
+    for (const RingTile& t : kRingTiles) {
+        const float us = b_dtype == SFG_I8 ? t.us_i8 : t.us_bf16;
+        if (us == 0.f || (glu && !t.glu) || (t.tile == kRingTileV && (!allow_v || k % 64 != 0))) continue;
+        const int64_t cols = glu ? t.bn / 2 : t.bn;
+        // grouped: half a tile of padding per group on average
+        const int64_t rows = (m + t.bm - 1) / t.bm + (groups > 1 ? groups / 2 : 0);
+        const int64_t tiles = rows * ((n + cols - 1) / cols);
+        for (int s = 1; s <= 16; ++s) {
+            const size_t part = s > 1 ? static_cast<size_t>(s) * m * nb * 4 : 0;
+            if (s > 1 && (!may_split || groups > 1 || t.tile == kRingTileV || n % 4 != 0 || slabs / s < 4 ||
+                          part > kRingMaxPart || part > workspace))
+                break;
+            const int64_t room = static_cast<int64_t>(kRingCus) * t.per_cu;
+            const float rounds = static_cast<float>((tiles * s + room - 1) / room);
+            // 3 us of prologue and epilogue a round; a split adds its reduce
+            // launch and one write and one read of the partials (4 TB/s)
+            float time = rounds * (static_cast<float>((slabs + s - 1) / s) * us + 3.f);
+            if (s > 1) time += 4.f + static_cast<float>(part) * 2.f / 4.0e6f;
+            if (best_us == 0.f || time < best_us) {
+                best_us = time;
+                best = RingPlan{t.tile, t.bm, t.bn, s, part};
+            }
+        }
+    }
+    return best;
+}
+
+namespace {
+
+template <int BDT, int BM, int BN, int NW, int NS>
+int launch_ring_tile(const TiledArgs& a, dim3 grid, int tm, int tn, int epi, float* part, hipStream_t s) {
+    constexpr bool kPairs = (BN / 64) % 2 == 0;  // GLU tiles pair gate and up blocks
+    const dim3 block(NW * 64);
+    if (part) {
+        if (epi == SFG_EPI_SWIGLU || epi == SFG_EPI_GLU_SILU_UP) {
+            if constexpr (kPairs) gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_SWIGLU, true><<<grid, block, 0, s>>>(a, tm, tn, part);
+            else return SFG_ERR_UNSUPPORTED;
+        } else {
+            gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_NONE, true><<<grid, block, 0, s>>>(a, tm, tn, part);
+        }
+        return SFG_OK;
+    }
+    switch (epi) {
+        case SFG_EPI_NONE: gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_NONE, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr); break;
+        case SFG_EPI_RESIDUAL: gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_RESIDUAL, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr); break;
+        case kEpiQkvRope:
+            if constexpr (BDT == SFG_BF16) {
+                gemm_ring_kernel<BDT, BM, BN, NW, NS, kEpiQkvRope, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr);
+                break;
+            } else {
+                return SFG_ERR_UNSUPPORTED;
+            }
+        default:
+            if constexpr (kPairs) {
+                if (epi == SFG_EPI_SWIGLU) gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_SWIGLU, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr);
+                else gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_GLU_SILU_UP, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr);
+                break;
+            } else {
+                return SFG_ERR_UNSUPPORTED;
+            }
+    }
+    return SFG_OK;
+}
+
+template <int BDT>
+int launch_ring_b(const TiledArgs& a, const RingPlan& plan, dim3 grid, int tm, int tn, int epi, float* part,
+                  hipStream_t s) {
+    switch (plan.tile) {
+        case kRingTile256x128: return launch_ring_tile<BDT, 256, 128, 8, 3>(a, grid, tm, tn, epi, part, s);
+        case kRingTile128x128: return launch_ring_tile<BDT, 128, 128, 8, 4>(a, grid, tm, tn, epi, part, s);
+        case kRingTile128x64: return launch_ring_tile<BDT, 128, 64, 4, 6>(a, grid, tm, tn, epi, part, s);
+        default: return launch_ring_tile<BDT, 64, 64, 4, 5>(a, grid, tm, tn, epi, part, s);
+    }
+}
+
+}  // namespace
+
+int launch_ring(const TiledArgs& a, const RingPlan& plan, int b_dtype, int epi, float* part, hipStream_t s) {
+    const bool glu = epi == SFG_EPI_SWIGLU || epi == SFG_EPI_GLU_SILU_UP;
+    const int64_t cols = glu ? plan.bn / 2 : plan.bn;
+    const int64_t tn = (a.n + cols - 1) / cols, tm = (a.m + plan.bm - 1) / plan.bm;
+    const dim3 grid = a.offsets ? dim3(static_cast<unsigned>(tn), static_cast<unsigned>(tm + a.groups))
+                                : dim3(static_cast<unsigned>(tm * tn), static_cast<unsigned>(plan.splits));
+    const int itm = a.offsets ? 0 : static_cast<int>(tm);
+    if (b_dtype == SFG_I8) return launch_ring_b<SFG_I8>(a, plan, grid, itm, static_cast<int>(tn), epi, part, s);
+    return launch_ring_b<SFG_BF16>(a, plan, grid, itm, static_cast<int>(tn), epi, part, s);
+}
+
+}  // namespace sfg

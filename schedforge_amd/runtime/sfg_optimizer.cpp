@@ -24,9 +24,9 @@ namespace {
 
 std::int64_t ceil_div(std::int64_t a, std::int64_t b) { return (a + b - 1) / b; }
 
-// The GEMM family's choice, restated from launch_gemm for the estimate:
-// skinny GEMV for few rows, the direct-to-LDS MFMA kernel for bf16 weights
-// and >= 1024 rows, the register-tiled MFMA kernel in between, VALU fp32.
+// The GEMM family's choice, simplified for the estimate: skinny GEMV for few
+// rows, the direct-to-LDS MFMA kernel for bf16 weights and >= 1024 rows, one
+// 128 x 128 tile rate in between, fp32.
 constexpr std::int64_t kSkinnyMaxRows = 64;
 constexpr std::int64_t kSkinnyGroupedMaxTotal = 512;
 constexpr std::int64_t kBigMinRows = 1024;
@@ -47,9 +47,9 @@ TileShape tile_shape(int tile) {
     }
 }
 
-// SFG_TILE_AUTO as the launcher resolves it: the largest tile with >= 512
-// workgroups (256 x 256 on the 64-k slab loop), and that tile for grouped
-// products from 128 workgroups up.
+// SFG_TILE_AUTO for the estimate: the largest tile with >= 512 workgroups
+// (256 x 256 on the 64-k slab loop), and that tile for grouped products from
+// 128 workgroups up.  (The launcher also weighs the ring tiles.)
 int auto_tile(std::int64_t m, std::int64_t n_out, bool glu, int groups) {
     if (groups > 1 && (ceil_div(m, 256) + groups) * ceil_div(n_out, glu ? 128 : 256) >= 128)
         return SFG_TILE_256x256_V;
