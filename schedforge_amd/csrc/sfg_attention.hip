@@ -2,8 +2,8 @@
 //
 //  * attn_prefill_rows_kernel: online softmax (attention_compiler.cpp:286-377),
 //    one wave per query row, 64 keys per step (one per lane), values
-//    accumulated with the wave owning the head dimension (up to 256): the
-//    fp32 path, and bf16 head dims the MFMA kernels do not lower.
+//    accumulated with the wave owning the head dimension (up to 256): fp32 and
+//    bf16 head dims the MFMA kernels (fp32: sfg_attention_f32.hip) do not lower.
 //  * attn_prefill_bf16_kernel: IO-aware flash prefill on v_mfma_f32_32x32x16_bf16.
 //    A workgroup owns 128 query rows of one (batch, head); each wave 32 rows.
 //    Scores are formed transposed, S^T = K Q^T, so lane l owns query row
@@ -27,8 +27,8 @@
 namespace sfg {
 
 // ===========================================================================
-// Row-per-wave prefill, any head_dim up to kRowMaxD: the fp32 path, and bf16
-// shapes the MFMA kernels do not lower (head_dim other than 64 / 128).
+// Row-per-wave prefill, any head_dim up to kRowMaxD: the fp32 and bf16 shapes
+// the MFMA kernels do not lower (head_dim other than 64 / 128).
 // ===========================================================================
 constexpr int kRowMaxD = 256;
 
@@ -191,8 +191,12 @@ int launch_attn_prefill_f32(const float* q, const float* k, const float* v, void
                             int64_t seq_q, int64_t seq_kv, int64_t head_dim, int causal,
                             float scale, hipStream_t stream) {
     if (head_dim > kRowMaxD) return SFG_ERR_UNSUPPORTED;
-    launch_prefill_rows(q, k, v, out, out_dtype, batch, q_heads, kv_heads, seq_q, seq_kv, head_dim,
-                        causal, scale, stream);
+    if (attn_prefill_f32_mfma_supported(q, k, v, out, batch, q_heads, seq_q, seq_kv, head_dim))
+        launch_attn_prefill_f32_mfma(q, k, v, out, out_dtype, batch, q_heads, kv_heads, seq_q, seq_kv, head_dim,
+                                     causal, scale, stream);
+    else
+        launch_prefill_rows(q, k, v, out, out_dtype, batch, q_heads, kv_heads, seq_q, seq_kv, head_dim,
+                            causal, scale, stream);
     return SFG_OK;
 }
 

@@ -25,9 +25,10 @@
 //  * gemm_mfma256_kernel, gemm_mfma_kernel  operands of 4 GiB and more, which
 //    the 32-bit offsets of the two above do not reach: 256x128 and 128x128
 //    tiles through padded LDS with register prefetch and 64-bit addresses.
-//  * gemm_vec_kernel      fp32 operands (the fp32 configurations) and the
-//    bf16 / int8 products the MFMA kernels do not lower: one sequential fp32
-//    FMA chain per output on the VALU.
+//  * fp32 operands: gemm_ring_kernel's and gemm_f32_small_kernel's fp32 MFMA
+//    forms (sfg_gemm_ring.hip).
+//  * gemm_vec_kernel      the products of any type the MFMA kernels do not
+//    lower: one sequential fp32 FMA chain per output on the VALU.
 #include <type_traits>
 
 #include "sfg_gemm_tile.hpp"
@@ -1766,6 +1767,20 @@ void launch_splitk_b(const SplitArgs& a, dim3 grid, bool tiled, hipStream_t s) {
     else gemm_splitk_kernel<BDT, false><<<grid, 256, 0, s>>>(a);
 }
 
+TiledArgs tiled_args(const GemmProblem& p, int groups) {
+    TiledArgs a{};
+    a.a = static_cast<const uint16_t*>(p.a); a.lda = p.lda; a.a_rows = p.a_rows;
+    a.a_rows_limit = p.a_rows ? p.a_rows_limit : p.m;
+    a.b = p.b; a.ldb = p.ldb; a.scales = p.b_dtype == SFG_F32 ? nullptr : p.b_scales;
+    a.b_group_stride = p.b_group_stride; a.s_group_stride = p.s_group_stride;
+    a.c = p.c; a.c_dtype = p.c_dtype; a.ldc = p.ldc;
+    a.residual = p.residual; a.ldr = p.ldr;
+    a.m = p.m; a.n = p.n; a.k = p.k; a.offsets = p.offsets; a.groups = groups;
+    a.qkv = p.qkv;
+    a.xcds = p.xcds;
+    return a;
+}
+
 // Sums split-K partials in slice order and applies the scales and epilogue.
 void launch_splitk_reduce(const GemmProblem& p, const float* part, int slices, int64_t nb, hipStream_t stream) {
     const SplitReduceArgs r{part, slices, p.b_scales, p.c, p.c_dtype, p.ldc, p.residual, p.ldr, p.m, p.n, nb};
@@ -1827,7 +1842,18 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
     if (p.epilogue == kEpiQkvRope && !gemm_qkv_rope_supported(p)) return SFG_ERR_UNSUPPORTED;
     if (p.a_dtype == SFG_F32) {
         if (p.b_dtype != SFG_F32) return SFG_ERR_UNSUPPORTED;
-        return launch_vec(p, stream);
+        // the fp32 MFMA kernels read 16-byte chunks of k; other depths, rows
+        // and operands of 4 GiB and more run on the VALU kernel
+        const int64_t a_rows = p.a_rows ? p.a_rows_limit : p.m;
+        const bool vec16 = ((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b)) & 15) == 0 &&
+                           p.lda % 4 == 0 && p.ldb % 4 == 0 && p.k % 4 == 0;
+        if (!vec16 || p.b_layout != SFG_LAYOUT_NK || p.b_group_stride % 4 != 0 ||
+            !fits_32bit(a_rows, p.lda, 4, glu ? 2 * p.n : p.n, p.ldb, 4, 2 * p.k))
+            return launch_vec(p, stream);
+        const int groups = p.offsets ? p.groups : 1;
+        // one pass over K whatever the rows: no split
+        const RingPlan plan = ring_plan(SFG_F32, p.m, p.n, p.k, glu, groups, false, false, 0);
+        return launch_ring(tiled_args(p, groups), plan, SFG_F32, p.epilogue, nullptr, stream);
     }
     if (p.a_dtype != SFG_BF16 || (p.b_dtype != SFG_BF16 && p.b_dtype != SFG_I8))
         return SFG_ERR_UNSUPPORTED;
@@ -1902,16 +1928,7 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
     // the 256 x 128 register-staged kernel needs whole tiles.
     const bool whole_n = p.n % (glu ? 64 : 128) == 0;
     const bool big = p.k % kGK == 0 && p.m >= kBigMinRows;
-    TiledArgs a{};
-    a.a = static_cast<const uint16_t*>(p.a); a.lda = p.lda; a.a_rows = p.a_rows;
-    a.a_rows_limit = p.a_rows ? p.a_rows_limit : p.m;
-    a.b = p.b; a.ldb = p.ldb; a.scales = p.b_scales;
-    a.b_group_stride = p.b_group_stride; a.s_group_stride = p.s_group_stride;
-    a.c = p.c; a.c_dtype = p.c_dtype; a.ldc = p.ldc;
-    a.residual = p.residual; a.ldr = p.ldr;
-    a.m = p.m; a.n = p.n; a.k = p.k; a.offsets = p.offsets; a.groups = groups;
-    a.qkv = p.qkv;
-    a.xcds = p.xcds;
+    const TiledArgs a = tiled_args(p, groups);
     if (fits_32bit(a.a_rows_limit, p.lda, 2, nb, p.ldb, p.b_dtype == SFG_I8 ? 1 : 2, p.k)) {
         // A plan that names a direct-to-LDS tile gets it (bf16, >= 1024 rows);
         // otherwise the ring tiles and the 256 x 256 one compete.  From 1024

@@ -42,7 +42,8 @@ struct TiledArgs {
 // product, kRingTileV standing for the 256 x 256 64-k-slab tile of
 // gemm_dma_kernel.  `part` bytes of split-K partial sums ([splits][m][B rows]
 // fp32) come from the caller's workspace.
-enum { kRingTileV = 1, kRingTile256x128, kRingTile128x128, kRingTile128x64, kRingTile64x64 };
+enum { kRingTileV = 1, kRingTile256x128, kRingTile128x128, kRingTile128x64, kRingTile64x64,
+       kRingTileSmall /* fp32 only: gemm_f32_small_kernel */ };
 constexpr size_t kRingNoLimit = ~size_t(0);
 struct RingPlan {
     int tile, bm, bn, splits;

@@ -80,6 +80,13 @@ int launch_attn_prefill_f32(const float* q, const float* k, const float* v, void
                              int out_dtype, int64_t batch, int64_t q_heads, int64_t kv_heads,
                              int64_t seq_q, int64_t seq_kv, int64_t head_dim, int causal,
                              float scale, hipStream_t stream);
+// The fp32 prefill's MFMA form (sfg_attention_f32.hip), which launch_attn_prefill_f32
+// takes where it is supported.
+bool attn_prefill_f32_mfma_supported(const float* q, const float* k, const float* v, const void* out,
+                                     int64_t batch, int64_t q_heads, int64_t seq_q, int64_t seq_kv, int64_t head_dim);
+void launch_attn_prefill_f32_mfma(const float* q, const float* k, const float* v, void* out, int out_dtype,
+                                  int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q, int64_t seq_kv,
+                                  int64_t head_dim, int causal, float scale, hipStream_t stream);
 // MFMA flash prefill at head_dim 64 / 128; other head dims up to 256 run the
 // row-per-wave kernel on the bf16 operands.
 int launch_attn_prefill_bf16(const uint16_t* q, const uint16_t* k, const uint16_t* v, void* out,
