@@ -302,8 +302,10 @@ int sfg_hip_attn_decode_paged_noalloc_v1(const float* q, const uint16_t* k_pool,
  * so seq_q = 1 sees all of them.  A row with no visible key comes out NaN, as
  * the reference's 0 / 0.  The MFMA split kernel takes the shapes it lowers
  * (bf16, head_dim 64 / 128, 16-token pages, one row, GQA group up to 16);
- * the rest run one wave per (sequence, row, head, split) with fp32 dot
- * products over the head dimension and an fp32 online softmax.  Errors:
+ * other bf16 shapes with that head_dim and page size run an MFMA kernel that
+ * keeps Q and the probabilities at fp32 precision; the rest one wave per
+ * (sequence, row, head, split) with fp32 dot products over the head dimension
+ * and an fp32 online softmax.  Errors:
  * SFG_ERR_INVALID_CONFIG for causal with seq_q > max_context (validate_config,
  * attention_compiler.cpp:23-29), SFG_ERR_UNSUPPORTED for head_dim > 256. */
 size_t sfg_hip_attn_paged_workspace_v1(int64_t batch, int64_t q_heads, int64_t kv_heads,

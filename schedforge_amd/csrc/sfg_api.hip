@@ -72,12 +72,14 @@ int check_decode_args(const float* q, const void* k_pool, const void* v_pool,
 
 // Which decode kernel a paged-attention call runs and its split count: the
 // MFMA split-KV kernel where it lowers the shape, else the row kernel (any
-// head_dim <= 256, page size, new-token count and pool dtype).  `bytes` is
-// the partials' workspace.
+// head_dim <= 256, page size, new-token count and pool dtype), in its
+// matrix-core form (rows_mfma) where that takes the shape.  `bytes` is the
+// partials' workspace; both forms of the row kernel leave the same partials.
 struct DecodePlan {
     bool mfma;
     int splits;
     size_t bytes;
+    bool rows_mfma = false;
 };
 
 DecodePlan plan_decode(int kv_dtype, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
@@ -87,6 +89,10 @@ DecodePlan plan_decode(int kv_dtype, int64_t batch, int64_t q_heads, int64_t kv_
         return {true, s, sfg::decode_workspace_bytes(batch, q_heads, head_dim, s)};
     }
     const int64_t rows = batch * seq_q * q_heads;
+    if (sfg::paged_mfma_rows_supported(kv_dtype, head_dim, page_tokens)) {
+        const int s = sfg::paged_mfma_rows_split_count(batch, q_heads, kv_heads, seq_q, head_dim, max_context, kv_splits);
+        return {false, s, sfg::paged_rows_workspace_bytes(rows, head_dim, s), true};
+    }
     const int s = sfg::paged_rows_split_count(rows, max_context, kv_splits);
     return {false, s, sfg::paged_rows_workspace_bytes(rows, head_dim, s)};
 }
@@ -118,6 +124,7 @@ int launch_paged(const DecodePlan& plan, const float* q, const void* k_pool, con
         a.batch = batch; a.q_heads = q_heads; a.kv_heads = kv_heads; a.seq_q = seq_q;
         a.head_dim = head_dim; a.page_tokens = page_tokens; a.pages_per_seq = pages_per_seq;
         a.num_pages = num_pages; a.splits = plan.splits; a.causal = causal; a.scale = sc;
+        a.mfma = plan.rows_mfma;
         rc = sfg::launch_attn_paged_rows(a, ws, as_stream(stream));
     }
     if (rc != SFG_OK)
@@ -523,7 +530,11 @@ size_t sfg_hip_attn_decode_workspace_v1(int64_t batch, int64_t q_heads, int64_t 
     const int s = sfg::decode_split_count(batch, 1, max_context, page_tokens, kv_splits);
     const size_t mfma = sfg::decode_workspace_bytes(batch, q_heads, head_dim, s);
     const int rs = sfg::paged_rows_split_count(batch * q_heads, max_context, kv_splits);
-    const size_t rows = sfg::paged_rows_workspace_bytes(batch * q_heads, head_dim, rs);
+    size_t rows = sfg::paged_rows_workspace_bytes(batch * q_heads, head_dim, rs);
+    // the row kernel's matrix-core form splits most at one kv head
+    const int ms = sfg::paged_mfma_rows_split_count(batch, q_heads, 1, 1, head_dim, max_context, kv_splits);
+    const size_t rows_mfma = sfg::paged_rows_workspace_bytes(batch * q_heads, head_dim, ms);
+    if (rows_mfma > rows) rows = rows_mfma;
     return mfma > rows ? mfma : rows;
 }
 
@@ -1127,6 +1138,7 @@ int sfg_hip_decoder_layer_v1(const sfg_layer_desc* d, const sfg_layer_weights* w
             a.head_dim = D; a.page_tokens = d->page_tokens; a.pages_per_seq = d->pages_per_seq;
             a.num_pages = d->num_pages; a.splits = plan.splits; a.causal = d->causal; a.scale = scale;
             a.mid_event = mid;
+            a.mfma = plan.rows_mfma;
             rc = sfg::launch_attn_paged_rows(a, b.attn_ws, s);
         }
         if (rc != SFG_OK) return fail(rc, "decode attention not lowered (head_dim %lld)", (long long)D);

@@ -19,6 +19,7 @@
 //    once; scores and the value product run on MFMA (see below), pages are
 //    double-buffered in registers, waves merge in LDS, splits merge in a
 //    second small kernel.
+#include <algorithm>
 #include <cstdlib>
 #include <type_traits>
 
@@ -1097,9 +1098,8 @@ int launch_attn_decode_paged(const float* q, int64_t q_row_stride, const float* 
 // Generic paged attention: any head_dim up to kRowMaxD, any page size, seq_q
 // >= 1 new query rows per sequence under the causal offset j <= len - seq_q +
 // i (attention_compiler.cpp:68-72), fp32 or bf16 pools; the decode path for
-// the shapes the MFMA split kernel does not lower (fp32 caches, head dims
-// other than 64 / 128, pages other than 16 tokens, more than one new token,
-// GQA groups above 16).  One wave per (sequence, query row, query head,
+// the shapes the MFMA kernels do not lower (fp32 caches, head dims other than
+// 64 / 128, pages other than 16 tokens).  One wave per (sequence, query row, query head,
 // split): lane j scores key j of each 64-key chunk against the query held in
 // LDS (one sequential fp32 FMA chain over the head dimension), then the wave
 // accumulates p V with lane d owning dims d, d + 64, ... (online softmax,
@@ -1232,6 +1232,287 @@ __global__ __launch_bounds__(64) void attn_paged_rows_kernel(PagedRowsArgs p) {
     }
 }
 
+// ===========================================================================
+// Paged attention of several query rows per sequence on the matrix cores (bf16
+// pools, head_dim 64 / 128, 16-token pages): drafted tokens, the tail of a
+// prompt, and one-row steps whose GQA group the split kernel above does not
+// take.  The seq_q x group query rows of a (sequence, kv head) fill MFMA columns,
+// 16 per workgroup, so each K / V byte is read once per 16 rows instead of once
+// per row; four waves take a quarter of the split's pages each.
+//
+// Queries and probabilities are fp32 here (as in the row kernel, whose shapes
+// these are): each enters as three bf16 terms (x = hi + mid + lo, 24 bits), with
+// one MFMA per term into the same fp32 accumulators; K and V are bf16 already.
+// The pass is bound by HBM, not by the three-fold MFMA work: 8 sequences x 5
+// rows x 16 heads over 3000 tokens, 652 us on the row kernel, 15 here.
+//
+// A page holding keys hidden from some rows or past the sequence's end zeroes V
+// past the end, and takes its tokens one at a time if a hidden one is not
+// finite (0 * inf).
+// ===========================================================================
+struct Bf16x3 {
+    bf16x8 t[3];
+};
+__device__ __forceinline__ void split3(float v, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
+    hi = f32_to_bf16(v);
+    const float r = v - bf16_to_f32(hi);
+    mid = f32_to_bf16(r);
+    lo = f32_to_bf16(r - bf16_to_f32(mid));
+}
+
+template <int kDecD>
+__global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs p, int chunks) {
+    // 16-column blocks per workgroup; two leave one wave per SIMD (27.8 against
+    // 23.0 us on the shape above, though each K / V byte is then read once)
+    constexpr int NCB = 1;
+    constexpr int kKs = kDecD / 32, kDt = kDecD / 16;
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int lr = lane & 15, lg = lane >> 4;
+    const int split = blockIdx.x, b = blockIdx.z;
+    const int kvh = blockIdx.y / chunks, chunk = blockIdx.y % chunks;
+    const int G = p.q_heads / p.kv_heads;
+    const int rows = p.seq_q * G;
+    const int col0 = chunk * (16 * NCB);
+    const int capacity = p.pages_per_seq * kPageTok;
+    const int len0 = p.seq_lens ? p.seq_lens[b] : p.uniform_len;
+    const int len = max(min(len0 + p.len_extra, capacity), 0);
+    const int pages = (len + kPageTok - 1) / kPageTok;
+    const int sp_begin = static_cast<int>(static_cast<int64_t>(pages) * split / p.splits);
+    const int sp_end = static_cast<int>(static_cast<int64_t>(pages) * (split + 1) / p.splits);
+    const int n_sp = sp_end - sp_begin;
+    const int w_begin = sp_begin + n_sp * wave / 4;
+    const int w_end = sp_begin + n_sp * (wave + 1) / 4;
+    // keys that every row of the step sees
+    const int all_see = p.causal ? len - p.seq_q + 1 : len;
+
+    // column c of block cb: query row i = r / G of head kvh G + r % G
+    int kend[NCB];
+    Bf16x3 qf[NCB][kKs];
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) {
+        const int r = col0 + 16 * cb + lr;
+        const bool has = r < rows;
+        const int i = has ? r / G : 0, h = kvh * G + (has ? r % G : 0);
+        kend[cb] = !has ? 0 : max(p.causal ? min(len, len - p.seq_q + i + 1) : len, 0);
+        const float* qr = p.q + p.qs.at(b, i, h);
+        float4 qa[kKs], qc[kKs];
+        float2 rot[kKs][4];
+#pragma unroll
+        for (int s = 0; s < kKs; ++s) {
+            qa[s] = *reinterpret_cast<const float4*>(qr + 32 * s + 8 * lg);
+            qc[s] = *reinterpret_cast<const float4*>(qr + 32 * s + 8 * lg + 4);
+        }
+        const bool rotate = p.rope && p.rope_rows > 0;
+        if (rotate) {
+            const int pos = min(max((p.rope_pos >= 0 ? p.rope_pos : len0) + i, 0), p.rope_rows - 1);
+            const float2* t = p.rope + static_cast<int64_t>(pos) * (kDecD / 2) + 4 * lg;
+#pragma unroll
+            for (int s = 0; s < kKs; ++s)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) rot[s][e] = t[16 * s + e];
+        }
+#pragma unroll
+        for (int s = 0; s < kKs; ++s) {
+            float v[8] = {qa[s].x, qa[s].y, qa[s].z, qa[s].w, qc[s].x, qc[s].y, qc[s].z, qc[s].w};
+            if (rotate) {
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const float2 cs = rot[s][e];
+                    const float ev = v[2 * e], od = v[2 * e + 1];
+                    v[2 * e] = ev * cs.x - od * cs.y;
+                    v[2 * e + 1] = ev * cs.y + od * cs.x;
+                }
+            }
+            uint32_t w[3][4];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                uint16_t a[3], c[3];
+                split3(has ? v[2 * e] : 0.f, a[0], a[1], a[2]);
+                split3(has ? v[2 * e + 1] : 0.f, c[0], c[1], c[2]);
+#pragma unroll
+                for (int t = 0; t < 3; ++t) w[t][e] = static_cast<uint32_t>(a[t]) | (static_cast<uint32_t>(c[t]) << 16);
+            }
+#pragma unroll
+            for (int t = 0; t < 3; ++t) qf[cb][s].t[t] = as_bf16x8(make_uint4(w[t][0], w[t][1], w[t][2], w[t][3]));
+        }
+    }
+
+    floatx4 acc[NCB][kDt];
+    float m_run[NCB], l_run[NCB];
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) {
+        m_run[cb] = -INFINITY;
+        l_run[cb] = 0.f;
+#pragma unroll
+        for (int i = 0; i < kDt; ++i) acc[cb][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+    const int32_t* table = p.page_table + static_cast<int64_t>(b) * p.pages_per_seq;
+    const int64_t head_stride = static_cast<int64_t>(kPageTok) * kDecD;
+    const int64_t page_stride = head_stride * p.kv_heads;
+    const uint16_t* kpool = static_cast<const uint16_t*>(p.k_pool) + kvh * head_stride + lr * kDecD + 8 * lg;
+    const uint16_t* vpool = static_cast<const uint16_t*>(p.v_pool) + kvh * head_stride + lr * kPageTok + 4 * lg;
+    uint4 kb[kKs];
+    uint2 vb[kDt];
+    bool okb = false;
+    // page ids 64 at a time, one per lane, so a page's loads wait on no read of
+    // their own; an id outside the pool reads page 0 and shows no key
+    int ids = 0, ids_base = w_begin - 64;
+    auto load_page = [&](int pg) __attribute__((always_inline)) {
+        if (pg - ids_base >= 64) {  // wave-uniform
+            ids_base = pg;
+            ids = pg + lane < w_end ? table[pg + lane] : -1;
+        }
+        const int id = __builtin_amdgcn_readlane(ids, pg - ids_base);
+        okb = id >= 0 && id < p.num_pages;
+        const int64_t base = okb ? static_cast<int64_t>(id) * page_stride : 0;
+#pragma unroll
+        for (int s = 0; s < kKs; ++s) kb[s] = *reinterpret_cast<const uint4*>(kpool + base + 32 * s);
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) vb[dt] = *reinterpret_cast<const uint2*>(vpool + base + dt * 16 * kPageTok);
+    };
+    if (w_begin < w_end) load_page(w_begin);
+    for (int pg = w_begin; pg < w_end; ++pg) {
+        uint4 kc[kKs];
+        uint2 vc[kDt];
+#pragma unroll
+        for (int s = 0; s < kKs; ++s) kc[s] = kb[s];
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt) vc[dt] = vb[dt];
+        const bool ok = okb;
+        if (pg + 1 < w_end) load_page(pg + 1);
+        const int tok0 = pg * kPageTok + 4 * lg;  // this lane's four tokens
+        bool slow = false;
+        if (!ok || (pg + 1) * kPageTok > all_see) {  // wave-uniform
+            // tokens past the end (or of no page) are not data
+            bool bad = false;
+#pragma unroll
+            for (int dt = 0; dt < kDt; ++dt) {
+                uint32_t w[2] = {vc[dt].x, vc[dt].y};
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const uint32_t mask = 0xFFFFu << (16 * (e & 1));
+                    if (!ok || tok0 + e >= len) w[e >> 1] &= ~mask;
+                    const uint32_t expo = (w[e >> 1] >> (16 * (e & 1))) & 0x7F80u;
+                    bad |= expo == 0x7F80u;
+                }
+                vc[dt] = make_uint2(w[0], w[1]);
+            }
+            slow = __any(bad);
+        }
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+            // three independent chains, the small terms summed first
+            floatx4 st3[3] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+            for (int s = 0; s < kKs; ++s)
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    st3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kc[s]), qf[cb][s].t[t], st3[t], 0, 0, 0);
+            const floatx4 st = st3[0] + (st3[1] + st3[2]);
+            float sv[4];
+            float mx = -INFINITY;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                sv[r] = ok && tok0 + r < kend[cb] ? st[r] * p.scale : -INFINITY;
+                mx = fmaxf(mx, sv[r]);
+            }
+            mx = xor16_max(mx);
+            mx = xor32_max(mx);
+            const float m_new = fmaxf(m_run[cb], mx);
+            const float alpha = m_run[cb] == -INFINITY ? 0.f : expf(m_run[cb] - m_new);
+            float pv[4];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) pv[r] = sv[r] == -INFINITY ? 0.f : expf(sv[r] - m_new);
+            l_run[cb] = l_run[cb] * alpha + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
+            m_run[cb] = m_new;
+#pragma unroll
+            for (int dt = 0; dt < kDt; ++dt) acc[cb][dt] *= alpha;
+            if (!slow) {
+                uint16_t w[3][4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) split3(pv[r], w[0][r], w[1][r], w[2][r]);
+                short4v pb[3];
+#pragma unroll
+                for (int t = 0; t < 3; ++t)
+                    pb[t] = as_short4(make_uint2(static_cast<uint32_t>(w[t][0]) | (static_cast<uint32_t>(w[t][1]) << 16),
+                                                 static_cast<uint32_t>(w[t][2]) | (static_cast<uint32_t>(w[t][3]) << 16)));
+#pragma unroll
+                for (int t = 2; t >= 0; --t)
+#pragma unroll
+                    for (int dt = 0; dt < kDt; ++dt)
+                        acc[cb][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as_short4(vc[dt]), pb[t], acc[cb][dt], 0, 0, 0);
+            } else {
+                // token by token: lane (lr, t / 4) holds its probability, lane
+                // (4 lg + r, t / 4) V of this lane's dims
+#pragma unroll 1
+                for (int t = 0; t < kPageTok; ++t) {
+                    const float mine = (t & 3) == 0 ? pv[0] : (t & 3) == 1 ? pv[1] : (t & 3) == 2 ? pv[2] : pv[3];
+                    const float pt = __shfl(mine, 16 * (t >> 2) + lr, 64);
+                    const bool sees = ok && pg * kPageTok + t < kend[cb];
+#pragma unroll
+                    for (int dt = 0; dt < kDt; ++dt) {
+                        // (masked, not selected: a select between the two is turned into a
+                        // load from scratch memory, which would hold V for every page)
+                        const uint32_t hi = 0u - static_cast<uint32_t>((t >> 1) & 1);
+                        const uint32_t word = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & hi);
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) {
+                            const uint32_t w = __shfl(static_cast<int>(word), 16 * (t >> 2) + 4 * lg + r, 64);
+                            const float v = bf16_to_f32(static_cast<uint16_t>(w >> (16 * (t & 1))));
+                            if (sees) acc[cb][dt][r] = fmaf(pt, v, acc[cb][dt][r]);
+                        }
+                    }
+                }
+            }
+        }
+    }
+    // merge the four waves in LDS: acc[cb][dt][r] = O^T[dim 16 dt + 4 lg + r][column lr]
+    constexpr int kCols = 16 * NCB;
+    __shared__ float s_m[4][kCols], s_l[4][kCols];
+    __shared__ float s_acc[4][kCols][kDecD];
+#pragma unroll
+    for (int cb = 0; cb < NCB; ++cb) {
+        const float l = xor32_sum(xor16_sum(l_run[cb]));
+#pragma unroll
+        for (int dt = 0; dt < kDt; ++dt)
+            *reinterpret_cast<floatx4*>(&s_acc[wave][16 * cb + lr][16 * dt + 4 * lg]) = acc[cb][dt];
+        if (lg == 0) {
+            s_m[wave][16 * cb + lr] = m_run[cb];
+            s_l[wave][16 * cb + lr] = l;
+        }
+    }
+    __syncthreads();
+    for (int o = threadIdx.x; o < min(kCols, rows - col0) * kDecD; o += 256) {
+        const int c = o / kDecD, d = o % kDecD;
+        const int r = col0 + c, i = r / G, h = kvh * G + r % G;
+        float mm = -INFINITY;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) mm = fmaxf(mm, s_m[w][c]);
+        float ls = 0.f, as = 0.f;
+#pragma unroll
+        for (int w = 0; w < 4; ++w) {
+            if (s_m[w][c] == -INFINITY) continue;
+            const float wf = expf(s_m[w][c] - mm);
+            ls = fmaf(s_l[w][c], wf, ls);
+            as = fmaf(s_acc[w][c][d], wf, as);
+        }
+        if (p.splits == 1) {
+            const float v = as / ls;  // no visible key: 0 / 0, as the reference's softmax gives
+            const int64_t at = p.os.at(b, i, h) + d;
+            if (p.out_f32) static_cast<float*>(p.out)[at] = v;
+            else static_cast<uint16_t*>(p.out)[at] = f32_to_bf16(v);
+        } else {
+            const int64_t part = ((static_cast<int64_t>(b) * p.seq_q + i) * p.q_heads + h) * p.splits + split;
+            p.part_acc[part * kDecD + d] = as;
+            if (d == 0) {
+                p.part_ml[2 * part] = mm;
+                p.part_ml[2 * part + 1] = ls;
+            }
+        }
+    }
+}
+
 // merge_online over a row's splits: weights e^(m_s - M), output sum / L.
 __global__ __launch_bounds__(64) void attn_combine_rows_kernel(const float* __restrict__ part_ml,
                                                               const float* __restrict__ part_acc,
@@ -1244,20 +1525,33 @@ __global__ __launch_bounds__(64) void attn_combine_rows_kernel(const float* __re
     const int bi = static_cast<int>(slot / q_heads);
     const int64_t o0 = os.at(bi / seq_q, bi % seq_q, h);
     const int D = head_dim;
+    const float* ml = part_ml + 2 * slot * splits;
+    const float* pa = part_acc + slot * splits * D;
     float M = -INFINITY;
-    for (int s = 0; s < splits; ++s) M = fmaxf(M, part_ml[2 * (slot * splits + s)]);
+    for (int s0 = 0; s0 < splits; s0 += 64) M = fmaxf(M, s0 + lane < splits ? ml[2 * (s0 + lane)] : -INFINITY);
+    M = wave_max(M);
     float L = 0.f;
     float o[4] = {0.f, 0.f, 0.f, 0.f};
-    for (int s = 0; s < splits; ++s) {
-        const int64_t part = slot * splits + s;
-        const float ms = part_ml[2 * part];
-        if (ms == -INFINITY) continue;
-        const float w = expf(ms - M);
-        L = fmaf(part_ml[2 * part + 1], w, L);
+    // eight splits at a time, their loads all issued before the ordered sum (slots
+    // past the count re-read the last split and are left out)
+    constexpr int kBatch = 8;
+    for (int s0 = 0; s0 < splits; s0 += kBatch) {
+        float ms[kBatch], ls[kBatch], av[kBatch][4];
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-            const int d = lane + 64 * r;
-            if (d < D) o[r] = fmaf(w, part_acc[part * D + d], o[r]);
+        for (int e = 0; e < kBatch; ++e) {
+            const int64_t sc = min(s0 + e, splits - 1);
+            ms[e] = ml[2 * sc];
+            ls[e] = ml[2 * sc + 1];
+#pragma unroll
+            for (int r = 0; r < 4; ++r) av[e][r] = 64 * r < D ? pa[sc * D + min(lane + 64 * r, D - 1)] : 0.f;
+        }
+#pragma unroll
+        for (int e = 0; e < kBatch; ++e) {
+            if (s0 + e >= splits || ms[e] == -INFINITY) continue;  // wave-uniform
+            const float w = expf(ms[e] - M);
+            L = fmaf(ls[e], w, L);
+#pragma unroll
+            for (int r = 0; r < 4; ++r) o[r] = fmaf(w, av[e][r], o[r]);
         }
     }
 #pragma unroll
@@ -1282,6 +1576,31 @@ size_t paged_rows_workspace_bytes(int64_t rows, int64_t head_dim, int splits) {
     if (splits <= 1) return 0;
     const size_t parts = static_cast<size_t>(rows) * splits;
     return ((parts * 2 * sizeof(float) + 255) / 256) * 256 + ((parts * head_dim * sizeof(float) + 255) / 256) * 256;
+}
+
+// The kernel above, where it takes the shape; groups of more than 16 query heads
+// included.  Q is read as 16-byte vectors.
+bool paged_mfma_rows_supported(int kv_dtype, int64_t head_dim, int64_t page_tokens) {
+    return kv_dtype == SFG_BF16 && (head_dim == 128 || head_dim == 64) && page_tokens == kPageTok;
+}
+
+// Two workgroups per CU (what its registers allow at D = 128) while a split keeps
+// 8 pages (two per wave); never
+// more partials than the larger of the row kernel's and the library's scratch.
+int paged_mfma_rows_split_count(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q, int64_t head_dim,
+                                int64_t max_keys, int32_t requested) {
+    const int64_t pages = (max_keys + kPageTok - 1) / kPageTok;
+    if (requested > 0) return static_cast<int>(requested < pages ? requested : (pages > 0 ? pages : 1));
+    const int64_t rows = seq_q * (q_heads / kv_heads);
+    const int64_t base = batch * kv_heads * ((rows + 15) / 16);
+    const size_t room = std::max(SFG_DECODE_SCRATCH_BYTES, paged_rows_workspace_bytes(
+                                                                batch * seq_q * q_heads, head_dim,
+                                                                paged_rows_split_count(batch * seq_q * q_heads, max_keys, 0)));
+    int s = 1;
+    while (base * s < 512 && pages / (s * 2) >= 8 &&
+           paged_rows_workspace_bytes(batch * seq_q * q_heads, head_dim, s * 2) <= room)
+        s *= 2;
+    return s;
 }
 
 int launch_attn_paged_rows(const PagedRowsLaunch& a, void* workspace, hipStream_t stream) {
@@ -1309,7 +1628,19 @@ int launch_attn_paged_rows(const PagedRowsLaunch& a, void* workspace, hipStream_
     p.num_pages = static_cast<int>(a.num_pages); p.splits = a.splits; p.causal = a.causal;
     p.scale = a.scale;
     const dim3 grid(static_cast<unsigned>(rows), static_cast<unsigned>(a.splits));
-    if (a.kv_dtype == SFG_F32) attn_paged_rows_kernel<float><<<grid, 64, 0, stream>>>(p);
+    // the matrix-core form reads Q and K as 16-byte vectors and V as 8-byte ones
+    const bool aligned = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k_pool)) & 15) == 0 &&
+                         (reinterpret_cast<uintptr_t>(a.v_pool) & 7) == 0 && a.q_stride_b % 4 == 0 &&
+                         a.q_stride_i % 4 == 0 && a.q_stride_h % 4 == 0;
+    const int64_t cols = a.seq_q * (a.q_heads / a.kv_heads);
+    const int64_t chunks64 = (cols + 15) / 16;
+    if (a.mfma && aligned && a.kv_heads * chunks64 <= 65535 && a.batch <= 65535) {
+        const int chunks = static_cast<int>(chunks64);
+        const dim3 mgrid(static_cast<unsigned>(a.splits), static_cast<unsigned>(a.kv_heads * chunks),
+                         static_cast<unsigned>(a.batch));
+        if (a.head_dim == 128) attn_paged_mfma_rows_kernel<128><<<mgrid, 256, 0, stream>>>(p, chunks);
+        else attn_paged_mfma_rows_kernel<64><<<mgrid, 256, 0, stream>>>(p, chunks);
+    } else if (a.kv_dtype == SFG_F32) attn_paged_rows_kernel<float><<<grid, 64, 0, stream>>>(p);
     else attn_paged_rows_kernel<uint16_t><<<grid, 64, 0, stream>>>(p);
     if (a.mid_event) (void)hipEventRecord(a.mid_event, stream);
     if (a.splits > 1)

@@ -134,7 +134,11 @@ struct PagedRowsLaunch {
     int64_t batch, q_heads, kv_heads, seq_q, head_dim, page_tokens, pages_per_seq, num_pages;
     int splits, causal; float scale;
     hipEvent_t mid_event;                   // recorded between the split and combine kernels
+    bool mfma;                              // the matrix-core form (paged_mfma_rows_supported)
 };
+bool paged_mfma_rows_supported(int kv_dtype, int64_t head_dim, int64_t page_tokens);
+int paged_mfma_rows_split_count(int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q, int64_t head_dim,
+                                int64_t max_keys, int32_t requested);
 int paged_rows_split_count(int64_t rows, int64_t max_keys, int32_t requested);
 size_t paged_rows_workspace_bytes(int64_t rows, int64_t head_dim, int splits);
 int launch_attn_paged_rows(const PagedRowsLaunch& a, void* workspace, hipStream_t stream);

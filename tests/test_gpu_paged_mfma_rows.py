@@ -1,0 +1,103 @@
+"""Paged attention of several query rows per sequence on the matrix cores (GPU
+only): column-block edges (1 .. 70 rows per kv head), GQA groups the one-row
+kernel does not take, both head dims, ragged lengths with an empty sequence and
+rows that see no key, an unaligned query (the row kernel), 1 split to more than
+there are pages, and pool contents that no row may see: stale tokens past the
+end and hidden tokens that are not finite.
+
+Q and the probabilities keep fp32 precision, so the tolerance is the fp32 one:
+scores of D products (error sqrt(D) 2^-24 of their size), expf at 1 ulp, sums of
+positive terms -- 3e-6 of the largest output, four times what those add up to.
+"""
+from __future__ import annotations
+
+import ctypes
+
+import numpy as np
+import pytest
+
+import oracle
+from schedforge_amd import _abi
+from schedforge_amd._abi import BF16, F32
+
+from _helpers import KEEP_ALIVE, bf16_dev, dev, host, stream
+
+pytestmark = pytest.mark.gpu
+torch = pytest.importorskip("torch")
+PT = 16
+
+# (q heads, kv heads, rows, D, longest, causal, splits, unaligned, poison)
+CASES = [(4, 4, 2, 128, 33, 1, 0, False, False), (16, 4, 4, 128, 1000, 1, 0, False, True),
+         (16, 4, 5, 128, 300, 1, 3, False, True), (6, 2, 1, 64, 200, 1, 0, False, False),
+         (12, 2, 7, 64, 120, 1, 40, False, True), (35, 5, 10, 128, 90, 1, 2, False, True),
+         (4, 1, 3, 64, 50, 0, 1, False, False), (8, 2, 6, 128, 64, 1, 0, True, True),
+         (32, 1, 2, 128, 500, 1, 0, False, True)]
+
+
+@pytest.mark.parametrize("hq,hkv,sq,d,longest,causal,splits,unaligned,poison", CASES)
+def test_paged_rows_on_the_matrix_cores(hq, hkv, sq, d, longest, causal, splits, unaligned, poison):
+    lib = _abi.load()
+    rng = np.random.default_rng(hq * 7 + sq * 3 + longest)
+    lens = np.array([longest, 0, 1, max(1, sq - 1), rng.integers(1, longest + 1)], np.int32)
+    b, pps = len(lens), (longest + PT - 1) // PT
+    pages = b * pps + 3
+    table = rng.permutation(pages)[: b * pps].reshape(b, pps).astype(np.int32)
+    kp = oracle.round_bf16(rng.standard_normal((pages, hkv, PT, d)).astype(np.float32))
+    vp = oracle.round_bf16(rng.standard_normal((pages, hkv, d, PT)).astype(np.float32))
+    q = rng.standard_normal((b, hq, sq, d)).astype(np.float32)
+    rows_seen = np.full(b, sq)  # rows compared
+    if poison:
+        for n in range(b):
+            for t in range(lens[n], pps * PT):  # past the end: anything
+                kp[table[n, t // PT], :, t % PT] = np.nan
+                vp[table[n, t // PT], :, :, t % PT] = np.inf if t % 2 else np.nan
+            if lens[n] > sq > 1:  # the last key: only the last row sees it
+                t = lens[n] - 1
+                vp[table[n, t // PT], :, ::2, t % PT] = -np.inf
+                vp[table[n, t // PT], :, 1::2, t % PT] = np.nan
+                rows_seen[n] = sq - 1
+    ref = np.full((b, hq, sq, d), np.nan)
+    for n in range(b):
+        L = int(lens[n])
+        k = kp[table[n]].transpose(1, 0, 2, 3).reshape(hkv, -1, d)[:, :L].astype(np.float64)
+        v = vp[table[n]].transpose(1, 0, 3, 2).reshape(hkv, -1, d)[:, :L].astype(np.float64)
+        for h in range(hq):
+            for i in range(rows_seen[n]):
+                end = min(L, L - sq + i + 1) if causal else L
+                if end <= 0:
+                    continue
+                j = h * hkv // hq
+                s = (k[j, :end] @ q[n, h, i].astype(np.float64)) / np.sqrt(d)
+                p = np.exp(s - s.max())
+                ref[n, h, i] = (p / p.sum()) @ v[j, :end]
+    buf = torch.zeros(q.size + 4, device="cuda")
+    qd = buf[1:1 + q.size] if unaligned else buf[:q.size]
+    qd.copy_(dev(q).reshape(-1))
+    kd, vd, td, ld = bf16_dev(kp), bf16_dev(vp), dev(table), dev(lens)
+    out = torch.zeros((b, hq, sq, d), device="cuda")
+    ws = torch.full((max(1, lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, sq, d, BF16, longest, PT, splits)),), 255,
+                    dtype=torch.uint8, device="cuda")
+    KEEP_ALIVE.extend([buf, out, ws])
+    _abi.check(lib.sfg_hip_attn_paged_v1(
+        qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), BF16, td.data_ptr(), ld.data_ptr(), out.data_ptr(), F32, b, hq, hkv,
+        sq, d, PT, pps, pages, longest, int(causal and sq <= longest), splits, ctypes.c_float(0.0), 0, ws.data_ptr(),
+        ws.numel(), stream()))
+    torch.cuda.synchronize()
+    got = host(out)
+    for n in range(b):
+        g, r = got[n, :, :rows_seen[n]], ref[n, :, :rows_seen[n]]
+        np.testing.assert_array_equal(np.isnan(g), np.isnan(r), err_msg=f"sequence {n}")
+        if np.isfinite(r).any():
+            err = np.nanmax(np.abs(g - r)) / max(np.nanmax(np.abs(r)), 1e-6)
+            assert err < 3e-6, (n, err)
+
+
+def test_decode_workspace_covers_every_kv_head_count():
+    """The one-row workspace query, which is not told the kv head count."""
+    lib = _abi.load()
+    for b, hq, ctx in ((1, 6, 5000), (4, 24, 900), (16, 48, 4096)):
+        top = lib.sfg_hip_attn_decode_workspace_v1(b, hq, 128, ctx, PT, 0)
+        for hkv in range(1, hq + 1):
+            if hq % hkv == 0:
+                need = lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, 1, 128, BF16, ctx, PT, 0)
+                assert need <= top, (b, hq, hkv, need, top)
