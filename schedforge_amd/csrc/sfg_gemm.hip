@@ -1803,14 +1803,27 @@ bool fits_32bit(int64_t a_rows, int64_t lda, int a_elem, int64_t b_rows, int64_t
 }
 }  // namespace
 
+// The tile launch_gemm gives a product on the ring / 256 x 256 kernels.
+// (int8: the QKV epilogue of a 128 x 128 wave block does not fit the registers.)
+RingPlan tile_plan(const GemmProblem& p, bool glu, int groups, bool split, size_t workspace_bytes) {
+    return ring_plan(p.b_dtype, p.m, p.n, p.k, glu, groups, split, p.b_dtype == SFG_BF16 || p.epilogue != kEpiQkvRope,
+                     workspace_bytes);
+}
+
 bool gemm_qkv_rope_supported(const GemmProblem& p) {
     const QkvRopeOut& o = p.qkv;
-    return p.a_dtype == SFG_BF16 && p.b_dtype == SFG_BF16 && !p.offsets && !p.a_rows &&
-           p.b_layout == SFG_LAYOUT_NK && p.m > kSkinnyMaxRows && p.k % kTK == 0 && o.rope && o.q &&
-           o.k && o.vt && o.seq > 0 && o.seq % 4 == 0 && p.m % o.seq == 0 && o.q_heads > 0 &&
-           o.kv_heads > 0 && p.n == (static_cast<int64_t>(o.q_heads) + 2 * o.kv_heads) * 128 &&
-           o.ld_vt % 64 == 0 && o.ld_vt >= o.seq &&
-           fits_32bit(p.m, p.lda, 2, p.n, p.ldb, 2, p.k);
+    if (!(p.a_dtype == SFG_BF16 && (p.b_dtype == SFG_BF16 || (p.b_dtype == SFG_I8 && p.b_scales)) && !p.offsets &&
+          !p.a_rows && p.b_layout == SFG_LAYOUT_NK && p.m > kSkinnyMaxRows && p.k % kTK == 0 && o.rope && o.q && o.k &&
+          o.vt && o.seq >= 4 && p.m % o.seq == 0 && o.q_heads > 0 && o.kv_heads > 0 &&
+          p.n == (static_cast<int64_t>(o.q_heads) + 2 * o.kv_heads) * 128 && o.ld_vt % 64 == 0 && o.ld_vt >= o.seq &&
+          fits_32bit(p.m, p.lda, 2, p.n, p.ldb, p.b_dtype == SFG_I8 ? 1 : 2, p.k)))
+        return false;
+    // Sequences that are not whole runs of four rows: the ring tiles only.  A
+    // product large enough for the 256 x 256 tile loses more on a smaller one
+    // than the separate split + RoPE pass costs.
+    if (o.seq % 4 == 0) return true;
+    const bool named = p.b_dtype == SFG_BF16 && p.m >= kBigMinRows && p.tile > SFG_TILE_AUTO;
+    return !named && tile_plan(p, false, 1, false, 0).tile != kRingTileV;
 }
 
 int gemm_preferred_layout(int64_t rows, int64_t k, bool grouped) {
@@ -1828,7 +1841,7 @@ size_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
     for (const int dt : {SFG_BF16, SFG_I8})
         for (const bool glu : {false, true}) {
             if (glu && n % 2) continue;
-            const RingPlan r = ring_plan(dt, m, glu ? n / 2 : n, k, glu, 1, true, dt == SFG_BF16, kRingNoLimit);
+            const RingPlan r = ring_plan(dt, m, glu ? n / 2 : n, k, glu, 1, true, true, kRingNoLimit);
             if (r.part > most) most = r.part;
         }
     return most;
@@ -1938,9 +1951,8 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
         const bool split = !p.offsets && !p.a_rows && p.epilogue != kEpiQkvRope && p.m < kBigMinRows &&
                            workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
         RingPlan plan{};
-        if (!named)
-            plan = ring_plan(p.b_dtype, p.m, p.n, p.k, glu, groups, split, p.b_dtype == SFG_BF16, workspace_bytes);
-        if (!named && plan.tile != kRingTileV) {
+        if (!named) plan = tile_plan(p, glu, groups, split, workspace_bytes);
+        if (!named && (plan.tile != kRingTileV || p.b_dtype != SFG_BF16)) {
             float* const part = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
             const int rc = launch_ring(a, plan, p.b_dtype, p.epilogue, part, stream);
             if (rc == SFG_OK && part) launch_splitk_reduce(p, part, plan.splits, nb, stream);

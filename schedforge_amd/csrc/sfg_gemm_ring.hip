@@ -152,7 +152,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int til
     const int asw = (l32 >> 1) & 7, bsw = kI8 ? (l32 >> 2) & 3 : asw;
     // A and B fragments of step J, a quarter of the slab (int8: raw, both steps
     // of the 32-k group at even J)
-    uint4 fa[2][WM], fb[2][kI8 ? 1 : WN], fq[2][kI8 ? WN : 1];
+    uint4 fa[2][WM], fb[2][WN], fq[2][kI8 ? WN : 1];
     auto frags = [&](const uint16_t* st, auto j_c) __attribute__((always_inline)) {
         constexpr int J = decltype(j_c)::value;
         const int ca = kI8 ? 4 * (J >> 1) + 2 * khalf + (J & 1) : 2 * J + khalf;
@@ -174,7 +174,19 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int til
                     sb + (wn * (BN / 2) + i * 32 + l32) * kBRow + ((2 * J + khalf) ^ bsw) * 8);
         }
     };
-    auto mfmas = [&](auto j_c) __attribute__((always_inline)) {
+    // int8: the bf16 fragments of step J from the raw ones
+    auto convert = [&](auto j_c) __attribute__((always_inline)) {
+        constexpr int J = decltype(j_c)::value;
+        if constexpr (kI8) {
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const uint4 q = fq[(J >> 1) & 1][j];
+                fb[J & 1][j] = (J & 1) ? i8x8_to_bf16x8(q.z, q.w) : i8x8_to_bf16x8(q.x, q.y);
+            }
+        }
+    };
+    // MFMAs [q0, q1) of step J, row-major over the wave's tiles
+    auto mfmas = [&](auto j_c, int q0, int q1) __attribute__((always_inline)) {
         constexpr int J = decltype(j_c)::value;
         if constexpr (kF32) {
             // a lane's four consecutive k feed four MFMAs of two k each
@@ -190,55 +202,54 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int til
                         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(av), __uint_as_float(bv), acc[i][j], 0, 0, 0);
                     }
         } else {
-            bf16x8 b[WN];
 #pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                if constexpr (kI8) {
-                    const uint4 q = fq[(J >> 1) & 1][j];
-                    b[j] = (J & 1) ? as_bf16x8(i8x8_to_bf16x8(q.z, q.w)) : as_bf16x8(i8x8_to_bf16x8(q.x, q.y));
-                } else {
-                    b[j] = as_bf16x8(fb[J & 1][j]);
-                }
+            for (int q = 0; q < WM * WN; ++q) {
+                if (q < q0 || q >= q1) continue;
+                acc[q / WN][q % WN] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(fa[J & 1][q / WN]), as_bf16x8(fb[J & 1][q % WN]),
+                                                                              acc[q / WN][q % WN], 0, 0, 0);
             }
-#pragma unroll
-            for (int i = 0; i < WM; ++i)
-#pragma unroll
-                for (int j = 0; j < WN; ++j)
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(as_bf16x8(fa[J & 1][i]), b[j], acc[i][j], 0, 0, 0);
         }
     };
     using J0 = std::integral_constant<int, 0>;
     using J1 = std::integral_constant<int, 1>;
     using J2 = std::integral_constant<int, 2>;
     using J3 = std::integral_constant<int, 3>;
+    // Step J's MFMAs with the next step's fragments (of stage st) read and DMA
+    // instructions [I0, I1) issued under them; int8 fragments of the next step
+    // are converted under the second half.
+    auto step = [&](auto j_c, auto next_c, const uint16_t* st, uint16_t* prev, int64_t s, auto i0_c, auto i1_c)
+                    __attribute__((always_inline)) {
+        constexpr int I0 = decltype(i0_c)::value, I1 = decltype(i1_c)::value;
+        constexpr int kM = WM * WN * (kF32 ? 4 : 1), kR = WM + WN;
+        frags(st, next_c);
+        issue(prev, s + NS - 1, I0, I1);
+        if constexpr (kI8) {
+            constexpr int kH = kM / 2;
+            mfmas(j_c, 0, kH);
+            spread_reads_loads<kH, (kR + 1) / 2 * 2 <= kH ? kR : kH, I1 - I0>();
+            __builtin_amdgcn_sched_barrier(0);
+            convert(next_c);
+            mfmas(j_c, kH, kM);
+            spread_valu<kM - kH, 12 * WN>();
+        } else {
+            mfmas(j_c, 0, kM);
+            spread_reads_loads<kM, kR, I1 - I0>();
+        }
+        __builtin_amdgcn_sched_barrier(0);
+    };
     // One slab: each step's fragments are read under the step before it.  The
     // barrier that publishes slab s + 1 also retires every read of slab s, so
     // the next slab's DMA may overwrite that stage.  Every slab issues the same
     // number of loads (past the end it re-fetches the last one), so the wait is
     // always for all but the newest NS - 2 groups.
     auto slab = [&](int64_t s, const uint16_t* cur, uint16_t* prev, const uint16_t* next) __attribute__((always_inline)) {
-        constexpr int kM = WM * WN * (kF32 ? 4 : 1), kR = WM + WN, kL1 = (kLoads + 2) / 3, kL2 = (2 * kLoads + 2) / 3;
-        frags(cur, J1{});
-        issue(prev, s + NS - 1, 0, kL1);
-        mfmas(J0{});
-        spread_reads_loads<kM, kR, kL1>();
-        __builtin_amdgcn_sched_barrier(0);
-        frags(cur, J2{});
-        issue(prev, s + NS - 1, kL1, kL2);
-        mfmas(J1{});
-        spread_reads_loads<kM, kR, kL2 - kL1>();
-        __builtin_amdgcn_sched_barrier(0);
-        frags(cur, J3{});
-        issue(prev, s + NS - 1, kL2, kLoads);
-        mfmas(J2{});
-        spread_reads_loads<kM, kR, kLoads - kL2>();
-        __builtin_amdgcn_sched_barrier(0);
+        constexpr int kL1 = (kLoads + 2) / 3, kL2 = (2 * kLoads + 2) / 3;
+        step(J0{}, J1{}, cur, prev, s, std::integral_constant<int, 0>{}, std::integral_constant<int, kL1>{});
+        step(J1{}, J2{}, cur, prev, s, std::integral_constant<int, kL1>{}, std::integral_constant<int, kL2>{});
+        step(J2{}, J3{}, cur, prev, s, std::integral_constant<int, kL2>{}, std::integral_constant<int, kLoads>{});
         wait_vmem_lds<(NS - 2) * kLoads>();
         barrier_no_fence();
-        frags(next, J0{});
-        mfmas(J3{});
-        spread_reads_loads<kM, kR, 0>();
-        __builtin_amdgcn_sched_barrier(0);
+        step(J3{}, J0{}, next, prev, s, std::integral_constant<int, kLoads>{}, std::integral_constant<int, kLoads>{});
     };
     issue(s0, slab0, 0, kLoads);
     issue(s1, slab0 + 1, 0, kLoads);
@@ -248,6 +259,7 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int til
     wait_vmem_lds<(NS - 2) * kLoads>();
     barrier_no_fence();
     frags(s0, J0{});
+    convert(J0{});
     int64_t s = slab0;
     if constexpr (NS == 3) {
         for (; s + 3 <= slab1; s += 3) {
@@ -314,11 +326,35 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int til
                 }
             }
     } else {
-        // 8 KB of staging per wave
+        if constexpr (kGlu && WM == 4 && WN == 4) {
+            if (p.c_dtype == SFG_BF16) {
+                // 16 KB of staging per wave; every wave's reads of the last
+                // slab are done before any wave reuses its stage
+                constexpr int kPer16 = kStage / 8192;
+                static_assert(NW <= 2 * kPer16, "staging fits two stage arrays");
+                wait_lds();
+                barrier_no_fence();
+                glu_epilogue_staged<EPI>(p, acc, row0 + wm * (BM / kWavesM), ncol0 + wn * (BN / 4), re, scales, lane,
+                                         (wave < kPer16 ? s0 : s1) + (wave % kPer16) * 8192);
+                return;
+            }
+        }
+        if constexpr (EPI == kEpiQkvRope && kI8) {
+            // the QKV epilogue takes finished products
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const float sc = scales[min(ncol0 + wn * (BN / 2) + j * 32 + l32, p.n - 1)];
+#pragma unroll
+                for (int i = 0; i < WM; ++i)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) acc[i][j][r] *= sc;
+            }
+        }
+        // 8 KB of staging per wave for the QKV epilogue of 64 x 64 wave blocks
         constexpr int kPer = kStage / 4096;  // waves' regions per stage array
-        static_assert(EPI != kEpiQkvRope || WM != WN || WM == 1 || NW <= 3 * kPer, "staging fits three stage arrays");
+        static_assert(EPI != kEpiQkvRope || WM != 2 || WN != 2 || NW <= 3 * kPer, "staging fits three stage arrays");
         float* const qkv_stage = reinterpret_cast<float*>((wave < kPer ? s0 : wave < 2 * kPer ? s1 : s2) + (wave % kPer) * 4096);
-        dma_tile_epilogue<BM, BN, NW, EPI, false, kWavesM>(p, acc, wm, wn, row0, ncol0, re, scales, qkv_stage);
+        dma_tile_epilogue<BM, BN, NW, EPI, false, kWavesM, true>(p, acc, wm, wn, row0, ncol0, re, scales, qkv_stage);
     }
 }
 
@@ -497,8 +533,8 @@ struct RingTile {
     bool glu;
 };
 constexpr RingTile kRingTiles[] = {
-    {kRingTileV, 256, 256, 1, 1.40f, 0.f, 0.f, true},
-    {kRingTile256x128, 256, 128, 1, 1.10f, 0.90f, 3.80f, true},
+    {kRingTileV, 256, 256, 1, 1.40f, 1.60f, 0.f, true},
+    {kRingTile256x128, 256, 128, 1, 1.10f, 1.05f, 3.80f, true},
     {kRingTile128x128, 128, 128, 1, 0.67f, 0.54f, 1.90f, true},
     {kRingTile128x64, 128, 64, 1, 0.45f, 0.42f, 1.00f, false},
     {kRingTile64x64, 64, 64, 2, 0.53f, 0.45f, 1.00f, false},
@@ -518,7 +554,8 @@ RingPlan ring_plan(int b_dtype, int64_t m, int64_t n, int64_t k, bool glu, int g
     float best_us = 0.f;
     for (const RingTile& t : kRingTiles) {
         float us = b_dtype == SFG_I8 ? t.us_i8 : b_dtype == SFG_F32 ? t.us_f32 : t.us_bf16;
-        if (us == 0.f || (glu && !t.glu) || (t.tile == kRingTileV && (!allow_v || k % 64 != 0))) continue;
+        if (us == 0.f || (glu && !t.glu) || (t.tile == kRingTileV && (!allow_v || (b_dtype == SFG_BF16 && k % 64 != 0))))
+            continue;
         const bool small = t.tile == kRingTileSmall;  // 32 output columns either way
         const int64_t cols = glu && !small ? t.bn / 2 : t.bn;
         if (small && glu) us *= 2.f;
@@ -564,7 +601,7 @@ int launch_ring_tile(const TiledArgs& a, dim3 grid, int tm, int tn, int epi, flo
         case SFG_EPI_NONE: gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_NONE, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr); break;
         case SFG_EPI_RESIDUAL: gemm_ring_kernel<BDT, BM, BN, NW, NS, SFG_EPI_RESIDUAL, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr); break;
         case kEpiQkvRope:
-            if constexpr (BDT == SFG_BF16) {
+            if constexpr (BDT != SFG_F32 && BM * BN < 256 * 256) {
                 gemm_ring_kernel<BDT, BM, BN, NW, NS, kEpiQkvRope, false><<<grid, block, 0, s>>>(a, tm, tn, nullptr);
                 break;
             } else {
@@ -586,6 +623,9 @@ template <int BDT>
 int launch_ring_b(const TiledArgs& a, const RingPlan& plan, dim3 grid, int tm, int tn, int epi, float* part,
                   hipStream_t s) {
     switch (plan.tile) {
+        case kRingTileV:  // bf16: gemm_dma_kernel's
+            if constexpr (BDT == SFG_I8) return part ? SFG_ERR_UNSUPPORTED : launch_ring_tile<BDT, 256, 256, 4, 3>(a, grid, tm, tn, epi, nullptr, s);
+            else return SFG_ERR_UNSUPPORTED;
         case kRingTile256x128: return launch_ring_tile<BDT, 256, 128, 8, 3>(a, grid, tm, tn, epi, part, s);
         case kRingTile128x128: return launch_ring_tile<BDT, 128, 128, 8, 4>(a, grid, tm, tn, epi, part, s);
         case kRingTile128x64: return launch_ring_tile<BDT, 128, 64, 4, 6>(a, grid, tm, tn, epi, part, s);

@@ -39,7 +39,7 @@ struct TiledArgs {
 };
 
 // The middle-size GEMM (sfg_gemm_ring.hip): tile and K split chosen for a
-// product, kRingTileV standing for the 256 x 256 64-k-slab tile of
+// product; with bf16 weights kRingTileV is the 256 x 256 64-k-slab tile of
 // gemm_dma_kernel.  `part` bytes of split-K partial sums ([splits][m][B rows]
 // fp32) come from the caller's workspace.
 enum { kRingTileV = 1, kRingTile256x128, kRingTile128x128, kRingTile128x64, kRingTile64x64,
@@ -135,6 +135,102 @@ __device__ __forceinline__ void qkv_rope_epilogue(const QkvRopeOut& o, const flo
     }
 }
 
+// The same for sequences of any length of at least four rows: a run of four rows
+// may end one and begin the next, and V^T takes single stores unless S % 4 == 0.
+// (Larger wave blocks than 64 x 64 have no registers for it.)
+template <int WM, int WN>
+__device__ __forceinline__ void qkv_rope_epilogue_any(const QkvRopeOut& o, const floatx16 (&acc)[WM][WN],
+                                                  int64_t wave_row0, int64_t wave_col0, int64_t re,
+                                                  int64_t n, int l32, int khalf) {
+    const int64_t H = static_cast<int64_t>(o.q_heads) * 128;
+    const int64_t kvd = static_cast<int64_t>(o.kv_heads) * 128;
+    const int seq = static_cast<int>(o.seq);
+#pragma unroll
+    for (int i = 0; i < WM; ++i) {
+        // One 32-row block: positions and (cos, sin) of all its rows and this
+        // lane's columns are fetched first, so the block waits for the table
+        // once instead of once per element.
+        int bq[4], sq[4];
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+            const int rr = static_cast<int>(wave_row0 + i * 32 + 8 * rq + 4 * khalf);
+            bq[rq] = rr / seq;
+            sq[rq] = rr - bq[rq] * seq;
+        }
+        // row e of a run of four: its (sequence, position), the run's own unless
+        // a sequence ends inside it (sequences hold at least four rows)
+        auto row_pos = [&](int rq, int e, int& b, int& sp) __attribute__((always_inline)) {
+            const bool wrap = sq[rq] + e >= seq;
+            b = bq[rq] + (wrap ? 1 : 0);
+            sp = sq[rq] + e - (wrap ? seq : 0);
+        };
+        float2 cs[WN][4][4];
+#pragma unroll
+        for (int j = 0; j < WN; ++j) {
+            const int64_t col = wave_col0 + j * 32 + l32;
+            const bool rot = col < H + kvd;  // uniform over the 32-column block
+            const int pr = static_cast<int>(col & 127) >> 1;
+#pragma unroll
+            for (int rq = 0; rq < 4; ++rq)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    int b, sp;
+                    row_pos(rq, e, b, sp);
+                    cs[j][rq][e] = rot ? o.rope[static_cast<int64_t>(sp) * 64 + pr] : make_float2(1.f, 0.f);
+                }
+        }
+#pragma unroll
+        for (int rq = 0; rq < 4; ++rq) {
+            const int64_t row = wave_row0 + i * 32 + 8 * rq + 4 * khalf;  // rows row .. row + 3
+#pragma unroll
+            for (int j = 0; j < WN; ++j) {
+                const int64_t col = wave_col0 + j * 32 + l32;
+                float v[4], pv[4];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    v[e] = acc[i][j][4 * rq + e];
+                    pv[e] = __shfl_xor(v[e], 1, 64);
+                }
+                if (col >= n || row >= re) continue;
+                const int d = static_cast<int>(col & 127);
+                if (col < H + kvd) {
+                    const bool isq = col < H;
+                    uint16_t* const base = isq ? o.q : o.k;
+                    const int64_t heads = isq ? o.q_heads : o.kv_heads;
+                    const int64_t head = isq ? col >> 7 : (col - H) >> 7;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        if (row + e >= re) break;
+                        int b, sp;
+                        row_pos(rq, e, b, sp);
+                        const float2 c = cs[j][rq][e];
+                        // (even, odd) -> (even c - odd s, odd c + even s), the same
+                        // fused operations as qkv_rope_epilogue_staged
+                        const float r0 = (d & 1) ? fmaf(v[e], c.x, pv[e] * c.y) : fmaf(v[e], c.x, -(pv[e] * c.y));
+                        base[((static_cast<int64_t>(b) * heads + head) * seq + sp) * 128 + d] = f32_to_bf16(r0);
+                    }
+                } else {
+                    const int64_t hv = (col - H - kvd) >> 7;
+                    if (seq % 4 == 0) {  // four positions of one sequence, 8-byte aligned
+                        uint2 pk;
+                        pk.x = pack_bf16x2(v[0], v[1]);
+                        pk.y = pack_bf16x2(v[2], v[3]);
+                        *reinterpret_cast<uint2*>(o.vt + ((static_cast<int64_t>(bq[rq]) * o.kv_heads + hv) * 128 + d) * o.ld_vt + sq[rq]) = pk;
+                    } else {
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if (row + e >= re) break;
+                            int b, sp;
+                            row_pos(rq, e, b, sp);
+                            o.vt[((static_cast<int64_t>(b) * o.kv_heads + hv) * 128 + d) * o.ld_vt + sp] = f32_to_bf16(v[e]);
+                        }
+                    }
+                }
+            }
+        }
+    }
+}
+
 // The same epilogue for a wave's block of a four-wave tile (128 x 128 of a
 // 256 x 256 tile, or 64 x 64 of a 128 x 128 one), through the wave's own LDS
 // stage array: for each 32-row block the accumulators go to LDS as fp32
@@ -145,7 +241,7 @@ __device__ __forceinline__ void qkv_rope_epilogue(const QkvRopeOut& o, const flo
 // A V^T block is staged transposed and leaves as 16-byte runs of positions; a
 // block past the last column, or V^T when the sequence length is not a
 // multiple of 8, takes the per-lane path.
-template <int WM, int WN>
+template <int WM, int WN, bool kAnySeq>
 __device__ __forceinline__ void qkv_rope_epilogue_staged(const QkvRopeOut& o, const floatx16 (&acc)[WM][WN],
                                                          int64_t wave_row0, int64_t wave_col0, int64_t re,
                                                          int64_t n, int lane, float* stage) {
@@ -157,7 +253,8 @@ __device__ __forceinline__ void qkv_rope_epilogue_staged(const QkvRopeOut& o, co
     const int64_t kvd = static_cast<int64_t>(o.kv_heads) * 128;
     const int64_t seq = o.seq;
     if (wave_col0 + kCols > n || (wave_col0 >= H + kvd && seq % 8 != 0)) {
-        qkv_rope_epilogue<WM, WN>(o, acc, wave_row0, wave_col0, re, n, l32, khalf);
+        if constexpr (kAnySeq) qkv_rope_epilogue_any<WM, WN>(o, acc, wave_row0, wave_col0, re, n, l32, khalf);
+        else qkv_rope_epilogue<WM, WN>(o, acc, wave_row0, wave_col0, re, n, l32, khalf);
         return;
     }
     const int col_in_head = static_cast<int>(wave_col0 & 127);  // 0, or 64 for 64-column blocks
@@ -396,6 +493,17 @@ __device__ __forceinline__ void spread_reads_loads() {
     }
 }
 
+// Scheduling groups for NM MFMAs with NV VALU instructions spread over them.
+template <int NM, int NV, int I = 0>
+__device__ __forceinline__ void spread_valu() {
+    if constexpr (I < NM) {
+        constexpr int here = (I + 1) * NV / NM - I * NV / NM;
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);                        // MFMA
+        if constexpr (here > 0) __builtin_amdgcn_sched_group_barrier(0x002, here, 0);  // VALU
+        spread_valu<NM, NV, I + 1>();
+    }
+}
+
 // Tile of this workgroup in a direct-to-LDS launch.  Grouped (p.offsets):
 // blockIdx.x is the column tile, blockIdx.y walks the row tiles of the groups
 // in order (group g: ceil(rows_g / BM) tiles; false past the last).  Dense: a
@@ -450,7 +558,7 @@ __device__ __forceinline__ bool dma_tile_coords(const TiledArgs& p, int tiles_m,
 // epilogue but the staged GLU one of the 64-k slab tile.  qkv_stage: this
 // wave's own LDS region for the staged QKV epilogue (every wave calls this
 // function: the staged path meets the others at a barrier first).
-template <int BM, int BN, int NW, int EPI, bool PP, int kWavesM = 2, int WM, int WN>
+template <int BM, int BN, int NW, int EPI, bool PP, int kWavesM = 2, bool kAnySeq = false, int WM, int WN>
 __device__ __forceinline__ void dma_tile_epilogue(const TiledArgs& p, const floatx16 (&acc)[WM][WN], int wm,
                                                   int wn, int64_t row0, int64_t ncol0, int64_t re,
                                                   const float* scales, float* qkv_stage) {
@@ -570,11 +678,12 @@ __device__ __forceinline__ void dma_tile_epilogue(const TiledArgs& p, const floa
             // reuses its array as staging (the DMA drained above)
             wait_lds();
             barrier_no_fence();
-            qkv_rope_epilogue_staged<WM, WN>(p.qkv, acc, row0 + wm * (BM / kWavesM), ncol0 + wn * (BN / kWavesN),
+            qkv_rope_epilogue_staged<WM, WN, kAnySeq>(p.qkv, acc, row0 + wm * (BM / kWavesM), ncol0 + wn * (BN / kWavesN),
                                              re, p.n, elane, qkv_stage);
         } else {
-            qkv_rope_epilogue<WM, WN>(p.qkv, acc, row0 + wm * (BM / kWavesM), ncol0 + wn * (BN / kWavesN), re,
-                                      p.n, el32, ekhalf);
+            const int64_t wrow0 = row0 + wm * (BM / kWavesM), wcol0 = ncol0 + wn * (BN / kWavesN);
+            if constexpr (kAnySeq) qkv_rope_epilogue_any<WM, WN>(p.qkv, acc, wrow0, wcol0, re, p.n, el32, ekhalf);
+            else qkv_rope_epilogue<WM, WN>(p.qkv, acc, wrow0, wcol0, re, p.n, el32, ekhalf);
         }
     }
 }

@@ -77,3 +77,24 @@ def test_ring_grouped_is_exact(counts, n, k, kind):
         torch.cuda.synchronize()
         acc = np.concatenate([arow[offsets[g]:offsets[g + 1]] @ bm[g].T for g in range(groups)])
         _check(out, F32, _epilogue(acc, epi, n).astype(np.float32), epi != EPI_NONE, f"{kind} {counts} epi {epi}")
+
+
+# the fused split + RoPE epilogue where sequences end inside a lane's run of four
+# rows: shortest sequences, one row past a tile, rows under and over 1024 (where a
+# named tile, or the 256 x 256 tile, takes the separate pass), int8
+@pytest.mark.parametrize("dtype,batch,seq", [("bf16", 40, 5), ("bf16", 3, 43), ("w8", 9, 29), ("w8", 2, 777),
+                                             ("bf16", 1, 1031), ("bf16", 5, 257), ("w8", 16, 4), ("bf16", 30, 3)])
+def test_qkv_epilogue_on_ragged_sequences(dtype, batch, seq):
+    import oracle
+    from schedforge_amd import CONFIGS
+    from schedforge_amd.layer import compile_decoder, execute_decoder_layer
+    from _helpers import TOL, decoder_data
+    cfg = CONFIGS["c4"].replace(batch=batch, sequence=seq, hidden=512, intermediate=1024, query_heads=4, kv_heads=2,
+                                dtype=dtype)
+    d = oracle.make_layer_data(cfg, 4100 + seq)
+    plan = compile_decoder(cfg, decoder_data(d), "cuda")
+    out = execute_decoder_layer(plan, d.input, warmup=0, repetitions=1).output
+    assert oracle.rel_error(out, oracle.decoder_layer(cfg, d)) < TOL[dtype]
+    if dtype == "bf16":  # the same bits as a tile named by the plan
+        plan.desc.gemm_tile = _abi.TILE_128x128
+        assert np.array_equal(execute_decoder_layer(plan, d.input, warmup=0, repetitions=1).output, out)
