@@ -64,11 +64,13 @@ int auto_tile(std::int64_t m, std::int64_t n_out, bool glu, int groups) {
 
 // The split-KV count the decode launcher picks when the policy leaves it open
 // (decode_split_count in the HIP library): double while the grid stays under
-// 1024 workgroups and each split keeps at least 32 pages.
+// 1024 workgroups and each split keeps at least 32 pages, then under 512
+// workgroups and 16 splits while each keeps 8.
 int auto_kv_splits(const DecoderConfig& c) {
     const std::int64_t pages = ceil_div(c.context_sequence, c.page_tokens);
     int s = 1;
     while (static_cast<std::int64_t>(c.batch) * c.kv_heads * s < 1024 && pages / (s * 2) >= 32) s *= 2;
+    while (s < 16 && static_cast<std::int64_t>(c.batch) * c.kv_heads * s < 512 && pages / (s * 2) >= 8) s *= 2;
     return s;
 }
 

@@ -101,3 +101,30 @@ def test_decode_workspace_covers_every_kv_head_count():
             if hq % hkv == 0:
                 need = lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, 1, 128, BF16, ctx, PT, 0)
                 assert need <= top, (b, hq, hkv, need, top)
+
+
+@pytest.mark.parametrize("b,hkv,longest", [(1, 8, 127), (1, 8, 129), (1, 8, 4096), (8, 8, 2000), (3, 2, 700)])
+def test_automatic_split_counts_match_one_split(b, hkv, longest):
+    """One-row steps of small batches, whose automatic split count keeps as few
+    as 8 pages a split: the same result as one split, within the rounding of the
+    probabilities to bf16 (2^-9 of a sum of positive weights)."""
+    lib = _abi.load()
+    rng = np.random.default_rng(longest)
+    hq, d, pps = 4 * hkv, 128, (longest + PT - 1) // PT
+    table = rng.permutation(b * pps).reshape(b, pps).astype(np.int32)
+    k, v = (bf16_dev(rng.standard_normal(s).astype(np.float32)) for s in ((b * pps, hkv, PT, d), (b * pps, hkv, d, PT)))
+    lens = np.full(b, longest, np.int32)
+    lens[-1] = max(1, longest // 9)
+    q, td, ld = dev(rng.standard_normal((b, hq, 1, d)).astype(np.float32)), dev(table), dev(lens)
+    outs = []
+    for splits in (0, 1):
+        n = lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, 1, d, BF16, longest, PT, splits)
+        out = torch.zeros((b, hq, d), device="cuda")
+        ws = torch.full((max(1, n),), 255, dtype=torch.uint8, device="cuda")
+        KEEP_ALIVE.extend([out, ws])
+        _abi.check(lib.sfg_hip_attn_paged_v1(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), BF16, td.data_ptr(), ld.data_ptr(), out.data_ptr(), F32, b, hq, hkv,
+            1, d, PT, pps, b * pps, longest, 1, splits, ctypes.c_float(0.0), 0, ws.data_ptr(), ws.numel(), stream()))
+        torch.cuda.synchronize()
+        outs.append(host(out))
+    np.testing.assert_allclose(outs[0], outs[1], atol=2.0 ** -8 * np.abs(outs[1]).max())
