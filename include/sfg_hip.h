@@ -175,7 +175,7 @@ int sfg_hip_rmsnorm_v1(const float* x, const float* w, void* y, int y_dtype, int
  * and for 65..1023 dense rows whose tiles alone leave compute units idle (at
  * most 64 MiB).  With a smaller workspace (or NULL) the same products run with
  * fewer splits or in a single pass.
- * b_layout SFG_LAYOUT_TILED is read by the decode GEMV only: bf16 / int8 B,
+ * b_layout SFG_LAYOUT_TILED is read by the decode kernels only: bf16 / int8 B,
  * at most 64 rows (grouped: 512 in all), K % 128 == 0 and N % 16 == 0;
  * other shapes with tiled B return SFG_ERR_UNSUPPORTED. */
 typedef struct {

@@ -1778,6 +1778,7 @@ TiledArgs tiled_args(const GemmProblem& p, int groups) {
     a.m = p.m; a.n = p.n; a.k = p.k; a.offsets = p.offsets; a.groups = groups;
     a.qkv = p.qkv;
     a.xcds = p.xcds;
+    a.b_tiled = p.b_layout == SFG_LAYOUT_TILED;
     return a;
 }
 
@@ -1804,10 +1805,11 @@ bool fits_32bit(int64_t a_rows, int64_t lda, int a_elem, int64_t b_rows, int64_t
 }  // namespace
 
 // The tile launch_gemm gives a product on the ring / 256 x 256 kernels.
-// (int8: the QKV epilogue of a 128 x 128 wave block does not fit the registers.)
+// (int8: the QKV epilogue of a 128 x 128 wave block does not fit the registers;
+// the bf16 256 x 256 tile reads [N][K] only.)
 RingPlan tile_plan(const GemmProblem& p, bool glu, int groups, bool split, size_t workspace_bytes) {
-    return ring_plan(p.b_dtype, p.m, p.n, p.k, glu, groups, split, p.b_dtype == SFG_BF16 || p.epilogue != kEpiQkvRope,
-                     workspace_bytes);
+    const bool allow_v = p.b_dtype == SFG_BF16 ? p.b_layout == SFG_LAYOUT_NK : p.epilogue != kEpiQkvRope;
+    return ring_plan(p.b_dtype, p.m, p.n, p.k, glu, groups, split, allow_v, workspace_bytes);
 }
 
 bool gemm_qkv_rope_supported(const GemmProblem& p) {
@@ -1907,8 +1909,18 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
     int nbt = g4 ? 4 : (glu ? 2 : (rows_hint <= 16 ? 1 : 2));
     if (!glu && !g4 && p.n % (16 * nbt) != 0) nbt = 1;  // widths of an odd number of 16-column tiles
     const int64_t tile_cols = glu ? 16 * nbt / 2 : 16 * nbt;
-    const bool skinny = skinny_rows && p.n % tile_cols == 0;
-    if (skinny_rows && !skinny && p.b_layout == SFG_LAYOUT_TILED) return SFG_ERR_UNSUPPORTED;
+    const bool tiled_ok = p.b_layout != SFG_LAYOUT_TILED || p.n % 16 == 0;
+    if (skinny_rows && p.n % tile_cols != 0 && p.b_layout == SFG_LAYOUT_TILED) return SFG_ERR_UNSUPPORTED;
+    // Grouped products of many rows per group: the ring tiles read each weight
+    // once, the skinny kernel once per 32 rows of a group.  Eight groups, W1|W3
+    // and W2 together, skinny against ring (us): bf16 H2048 I1408, 128 rows 45 /
+    // 47, 200 rows 56 / 49, 512 rows 110 / 62; H4096 I14336, 128 rows 506 / 538,
+    // 200 rows 649 / 546; int8 H4096 I14336, 200 rows 379 / 403, 256 rows 422 /
+    // 399, 512 rows 764 / 577; int8 H2048 I1408, 128 rows 39 / 39, 256 rows 65 / 41.
+    const int64_t ring_rows = p.b_dtype == SFG_I8 ? 28 : 20;  // rows per group
+    const bool ring_grouped = p.offsets && p.m >= ring_rows * groups && tiled_ok && fits_32bit(p.a_rows ? p.a_rows_limit : p.m, p.lda, 2, nb, p.ldb,
+                                                    p.b_dtype == SFG_I8 ? 1 : 2, p.k);
+    const bool skinny = skinny_rows && p.n % tile_cols == 0 && !ring_grouped;
     if (skinny) {
         const int mt = rows_hint <= 16 ? 1 : (rows_hint <= 32 ? 2 : 4);
         // A grouped launch already has groups x N/16 workgroups, several per
@@ -1936,7 +1948,8 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
         else launch_skinny_b<SFG_BF16>(a, grid, mt, nbt, waves, p.epilogue, tiled, stream);
         return SFG_OK;
     }
-    if (p.b_layout == SFG_LAYOUT_TILED) return SFG_ERR_UNSUPPORTED;  // tiled weights feed the skinny kernel only
+    // (fragment-tiled weights feed the skinny kernel and grouped ring products)
+    if (p.b_layout == SFG_LAYOUT_TILED && !(ring_grouped && skinny_rows)) return SFG_ERR_UNSUPPORTED;
     // The direct-to-LDS and 128 x 128 kernels mask a ragged last column tile;
     // the 256 x 128 register-staged kernel needs whole tiles.
     const bool whole_n = p.n % (glu ? 64 : 128) == 0;

@@ -13,7 +13,8 @@ namespace sfg {
 // keeps in flight.  The ring holds most of the CU's 160 KB for one workgroup
 // (NS - 1 slabs of 16 - 32 KB in flight), one barrier per 64 k.
 //
-// A rows are 128 B with 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7);
+// B rows come from [N][K] or from the fragment-tiled layout (the DMA lanes pick
+// their chunks).  A rows are 128 B with 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7);
 // bf16 B rows the same; int8 B rows are 64 B with chunk c in slot
 // c ^ ((r >> 2) & 3), converted to bf16 (exactly) between the LDS read and the
 // MFMA, under the matrix pipe.  The MFMA k order is free as long as A and B
@@ -115,6 +116,17 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int til
             const int64_t col = ncol0 + local;
             brow = col < p.n ? col : 0;
         }
+        if constexpr (!kF32) {
+            if (p.b_tiled) {
+                // 16-row x 128-k tiles: 16-byte chunk c of a row's 64-k half sits
+                // in (bf16) fragment c / 4, lane group c % 4; (int8) fragment
+                // c % 2, lane group c / 2
+                const int64_t at = (brow / 16) * (p.k / 128) * (2048 * kBElem) + (brow % 16) * 16 +
+                                   (kI8 ? (chunk & 1) * 1024 + (chunk >> 1) * 256 : (chunk >> 2) * 1024 + (chunk & 3) * 256);
+                b_off[i] = static_cast<uint32_t>(at);
+                continue;
+            }
+        }
         b_off[i] = static_cast<uint32_t>((brow * p.ldb) * kBElem + chunk * 16);
     }
     // DMA instructions [i0, i1) of slab s into stage st (A's first, then B's).
@@ -122,7 +134,8 @@ __global__ __launch_bounds__(NW * 64) void gemm_ring_kernel(TiledArgs p, int til
     auto issue = [&](uint16_t* st, int64_t s, int i0, int i1) __attribute__((always_inline)) {
         const int64_t sl = min(s, slab1 - 1);
         const bool tail = tail_a != 0 && sl == all_slabs - 1;  // wave-uniform
-        const uint32_t ka = static_cast<uint32_t>(sl * 128), kb = static_cast<uint32_t>(sl * kSlabK * kBElem);
+        const uint32_t ka = static_cast<uint32_t>(sl * 128), kb = !kF32 && p.b_tiled ? static_cast<uint32_t>((sl >> 1) * (2048 * kBElem) + (sl & 1) * (kI8 ? 512 : 2048))
+                                                                                      : static_cast<uint32_t>(sl * kSlabK * kBElem);
 #pragma unroll
         for (int i = 0; i < kLoadsA; ++i) {
             if (i < i0 || i >= i1) continue;
@@ -536,6 +549,7 @@ constexpr RingTile kRingTiles[] = {
     {kRingTileV, 256, 256, 1, 1.40f, 1.60f, 0.f, true},
     {kRingTile256x128, 256, 128, 1, 1.10f, 1.05f, 3.80f, true},
     {kRingTile128x128, 128, 128, 1, 0.67f, 0.54f, 1.90f, true},
+    {kRingTile64x128, 64, 128, 1, 0.46f, 0.35f, 1.00f, true},
     {kRingTile128x64, 128, 64, 1, 0.45f, 0.42f, 1.00f, false},
     {kRingTile64x64, 64, 64, 2, 0.53f, 0.45f, 1.00f, false},
     {kRingTileSmall, 32, 32, 1, 0.f, 0.f, 0.13f, true},
@@ -628,6 +642,7 @@ int launch_ring_b(const TiledArgs& a, const RingPlan& plan, dim3 grid, int tm, i
             else return SFG_ERR_UNSUPPORTED;
         case kRingTile256x128: return launch_ring_tile<BDT, 256, 128, 8, 3>(a, grid, tm, tn, epi, part, s);
         case kRingTile128x128: return launch_ring_tile<BDT, 128, 128, 8, 4>(a, grid, tm, tn, epi, part, s);
+        case kRingTile64x128: return launch_ring_tile<BDT, 64, 128, 4, 6>(a, grid, tm, tn, epi, part, s);
         case kRingTile128x64: return launch_ring_tile<BDT, 128, 64, 4, 6>(a, grid, tm, tn, epi, part, s);
         default: return launch_ring_tile<BDT, 64, 64, 4, 5>(a, grid, tm, tn, epi, part, s);
     }

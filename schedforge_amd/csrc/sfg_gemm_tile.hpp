@@ -36,13 +36,14 @@ struct TiledArgs {
     int groups;
     QkvRopeOut qkv;           // kEpiQkvRope only
     int xcds;                 // XCDs the dispatcher deals workgroups over
+    int b_tiled;              // gemm_ring_kernel: B in SFG_LAYOUT_TILED
 };
 
 // The middle-size GEMM (sfg_gemm_ring.hip): tile and K split chosen for a
 // product; with bf16 weights kRingTileV is the 256 x 256 64-k-slab tile of
 // gemm_dma_kernel.  `part` bytes of split-K partial sums ([splits][m][B rows]
 // fp32) come from the caller's workspace.
-enum { kRingTileV = 1, kRingTile256x128, kRingTile128x128, kRingTile128x64, kRingTile64x64,
+enum { kRingTileV = 1, kRingTile256x128, kRingTile128x128, kRingTile64x128, kRingTile128x64, kRingTile64x64,
        kRingTileSmall /* fp32 only: gemm_f32_small_kernel */ };
 constexpr size_t kRingNoLimit = ~size_t(0);
 struct RingPlan {

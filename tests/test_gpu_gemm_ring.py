@@ -14,7 +14,7 @@ import pytest
 from schedforge_amd import _abi
 from schedforge_amd._abi import BF16, EPI_GLU_SILU_UP, EPI_NONE, EPI_RESIDUAL, EPI_SWIGLU, F32
 
-from _helpers import KEEP_ALIVE, bf16_dev, dev, stream
+from _helpers import KEEP_ALIVE, bf16_dev, dev, host, stream, tile_nk
 from test_gpu_gemm_random import _args, _check, _epilogue, _weights
 
 pytestmark = pytest.mark.gpu
@@ -52,10 +52,12 @@ def test_ring_dense_is_exact(m, n, k, kind):
 
 
 # groups of no row, one row and one past a tile; ids outside A read zero rows
+# (layout 1: fragment-tiled weights, up to 512 rows in all)
 @pytest.mark.parametrize("kind", ["bf16", "i8"])
-@pytest.mark.parametrize("counts,n,k", [((0, 65, 1, 500), 64, 96), ((600, 0, 0, 129, 3), 192, 1376),
-                                        ((257, 300, 255, 1, 0, 64, 200), 1408, 160)])
-def test_ring_grouped_is_exact(counts, n, k, kind):
+@pytest.mark.parametrize("counts,n,k,layout", [((0, 65, 1, 500), 64, 96, 0), ((600, 0, 0, 129, 3), 192, 1376, 0),
+                                               ((257, 300, 255, 1, 0, 64, 200), 1408, 160, 0), ((0, 65, 1, 200), 64, 128, 1),
+                                               ((300, 0, 129, 3), 208, 384, 1), ((100, 412), 16, 1408, 1)])
+def test_ring_grouped_is_exact(counts, n, k, layout, kind):
     lib = _abi.load()
     rng = np.random.default_rng(n + k)
     groups, m, t = len(counts), sum(counts), 300
@@ -69,9 +71,12 @@ def test_ring_grouped_is_exact(counts, n, k, kind):
     for epi in (EPI_NONE, EPI_GLU_SILU_UP):
         nb = 2 * n if epi != EPI_NONE else n
         bd, b_dtype, sd, bm = _weights(rng, kind, (groups, nb), k, 0)
+        if layout:
+            w = host(bd).reshape(groups, nb, k)
+            bd = dev(np.stack([tile_nk(w[g], "int8" if kind == "i8" else "bf16") for g in range(groups)]))
         out = torch.full((m, n), 77, dtype=torch.float32, device="cuda")
         KEEP_ALIVE.append(out)
-        args = _args(bf16_dev(a), BF16, bd, b_dtype, sd, out, F32, None, m, n, k, epi, 0, 0)
+        args = _args(bf16_dev(a), BF16, bd, b_dtype, sd, out, F32, None, m, n, k, epi, layout, 0)
         _abi.check(lib.sfg_hip_gemm_grouped_v1(ctypes.byref(args), dev(rows).data_ptr(), t, dev(offsets).data_ptr(),
                                                groups, nb * k, nb if sd is not None else 0, None, 0, stream()))
         torch.cuda.synchronize()
