@@ -1104,8 +1104,8 @@ int launch_attn_decode_paged(const float* q, int64_t q_row_stride, const float* 
 // Generic paged attention: any head_dim up to kRowMaxD, any page size, seq_q
 // >= 1 new query rows per sequence under the causal offset j <= len - seq_q +
 // i (attention_compiler.cpp:68-72), fp32 or bf16 pools; the decode path for
-// the shapes the MFMA kernels do not lower (fp32 caches, head dims other than
-// 64 / 128, pages other than 16 tokens).  One wave per (sequence, query row, query head,
+// the shapes the MFMA kernels do not lower (head dims other than 64 / 128, pages
+// other than 16 tokens).  One wave per (sequence, query row, query head,
 // split): lane j scores key j of each 64-key chunk against the query held in
 // LDS (one sequential fp32 FMA chain over the head dimension), then the wave
 // accumulates p V with lane d owning dims d, d + 64, ... (online softmax,
@@ -1239,15 +1239,15 @@ __global__ __launch_bounds__(64) void attn_paged_rows_kernel(PagedRowsArgs p) {
 }
 
 // ===========================================================================
-// Paged attention of several query rows per sequence on the matrix cores (bf16
-// pools, head_dim 64 / 128, 16-token pages): drafted tokens, the tail of a
-// prompt, and one-row steps whose GQA group the split kernel above does not
-// take.  The seq_q x group query rows of a (sequence, kv head) fill MFMA columns,
+// Paged attention of several query rows per sequence on the matrix cores
+// (head_dim 64 / 128, 16-token pages): drafted tokens, the tail of a prompt,
+// one-row steps whose GQA group the split kernel above does not take, and all
+// steps over fp32 pools (v_mfma_f32_16x16x4_f32 in the same layout).  The seq_q x group query rows of a (sequence, kv head) fill MFMA columns,
 // 16 per workgroup, so each K / V byte is read once per 16 rows instead of once
 // per row; four waves take a quarter of the split's pages each.
 //
 // Queries and probabilities are fp32 here (as in the row kernel, whose shapes
-// these are): each enters as three bf16 terms (x = hi + mid + lo, 24 bits), with
+// these are): over bf16 pools each enters as three bf16 terms (x = hi + mid + lo, 24 bits), with
 // one MFMA per term into the same fp32 accumulators; K and V are bf16 already.
 // The pass is bound by HBM, not by the three-fold MFMA work: 8 sequences x 5
 // rows x 16 heads over 3000 tokens, 652 us on the row kernel, 15 here.
@@ -1266,12 +1266,16 @@ __device__ __forceinline__ void split3(float v, uint16_t& hi, uint16_t& mid, uin
     lo = f32_to_bf16(r - bf16_to_f32(mid));
 }
 
-template <int kDecD>
+template <typename KvT, int kDecD>
 __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs p, int chunks) {
     // 16-column blocks per workgroup; two leave one wave per SIMD (27.8 against
     // 23.0 us on the shape above, though each K / V byte is then read once)
     constexpr int NCB = 1;
-    constexpr int kKs = kDecD / 32, kDt = kDecD / 16;
+    constexpr bool kF32 = sizeof(KvT) == 4;
+    // k-steps of a page's scores as loaded: 16 bytes of K per lane, 32 (fp32: 16) dims
+    constexpr int kStep = kF32 ? 16 : 32, kKs = kDecD / kStep, kDt = kDecD / 16;
+    constexpr int kLane = kStep / 4;  // dims of a step per lane
+    using VecV = std::conditional_t<kF32, uint4, uint2>;  // four tokens of V
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int lr = lane & 15, lg = lane >> 4;
@@ -1294,7 +1298,8 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
 
     // column c of block cb: query row i = r / G of head kvh G + r % G
     int kend[NCB];
-    Bf16x3 qf[NCB][kKs];
+    Bf16x3 qf[NCB][kF32 ? 1 : kKs];
+    float4 qf32[NCB][kF32 ? kKs : 1];
 #pragma unroll
     for (int cb = 0; cb < NCB; ++cb) {
         const int r = col0 + 16 * cb + lr;
@@ -1302,45 +1307,51 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
         const int i = has ? r / G : 0, h = kvh * G + (has ? r % G : 0);
         kend[cb] = !has ? 0 : max(p.causal ? min(len, len - p.seq_q + i + 1) : len, 0);
         const float* qr = p.q + p.qs.at(b, i, h);
-        float4 qa[kKs], qc[kKs];
-        float2 rot[kKs][4];
+        float qv[kKs][kLane];
+        float2 rot[kKs][kLane / 2];
 #pragma unroll
-        for (int s = 0; s < kKs; ++s) {
-            qa[s] = *reinterpret_cast<const float4*>(qr + 32 * s + 8 * lg);
-            qc[s] = *reinterpret_cast<const float4*>(qr + 32 * s + 8 * lg + 4);
-        }
+        for (int s = 0; s < kKs; ++s)
+#pragma unroll
+            for (int e = 0; e < kLane; e += 4) {
+                const float4 t = *reinterpret_cast<const float4*>(qr + kStep * s + kLane * lg + e);
+                qv[s][e] = t.x; qv[s][e + 1] = t.y; qv[s][e + 2] = t.z; qv[s][e + 3] = t.w;
+            }
         const bool rotate = p.rope && p.rope_rows > 0;
         if (rotate) {
             const int pos = min(max((p.rope_pos >= 0 ? p.rope_pos : len0) + i, 0), p.rope_rows - 1);
-            const float2* t = p.rope + static_cast<int64_t>(pos) * (kDecD / 2) + 4 * lg;
+            const float2* t = p.rope + static_cast<int64_t>(pos) * (kDecD / 2) + kLane / 2 * lg;
 #pragma unroll
             for (int s = 0; s < kKs; ++s)
 #pragma unroll
-                for (int e = 0; e < 4; ++e) rot[s][e] = t[16 * s + e];
+                for (int e = 0; e < kLane / 2; ++e) rot[s][e] = t[kStep / 2 * s + e];
         }
 #pragma unroll
         for (int s = 0; s < kKs; ++s) {
-            float v[8] = {qa[s].x, qa[s].y, qa[s].z, qa[s].w, qc[s].x, qc[s].y, qc[s].z, qc[s].w};
+            float (&v)[kLane] = qv[s];
             if (rotate) {
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
+                for (int e = 0; e < kLane / 2; ++e) {
                     const float2 cs = rot[s][e];
                     const float ev = v[2 * e], od = v[2 * e + 1];
                     v[2 * e] = ev * cs.x - od * cs.y;
                     v[2 * e + 1] = ev * cs.y + od * cs.x;
                 }
             }
-            uint32_t w[3][4];
+            if constexpr (kF32) {
+                qf32[cb][s] = has ? make_float4(v[0], v[1], v[2], v[3]) : make_float4(0.f, 0.f, 0.f, 0.f);
+            } else {
+                uint32_t w[3][4];
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                uint16_t a[3], c[3];
-                split3(has ? v[2 * e] : 0.f, a[0], a[1], a[2]);
-                split3(has ? v[2 * e + 1] : 0.f, c[0], c[1], c[2]);
+                for (int e = 0; e < 4; ++e) {
+                    uint16_t a[3], c[3];
+                    split3(has ? v[2 * e] : 0.f, a[0], a[1], a[2]);
+                    split3(has ? v[2 * e + 1] : 0.f, c[0], c[1], c[2]);
 #pragma unroll
-                for (int t = 0; t < 3; ++t) w[t][e] = static_cast<uint32_t>(a[t]) | (static_cast<uint32_t>(c[t]) << 16);
+                    for (int t = 0; t < 3; ++t) w[t][e] = static_cast<uint32_t>(a[t]) | (static_cast<uint32_t>(c[t]) << 16);
+                }
+#pragma unroll
+                for (int t = 0; t < 3; ++t) qf[cb][s].t[t] = as_bf16x8(make_uint4(w[t][0], w[t][1], w[t][2], w[t][3]));
             }
-#pragma unroll
-            for (int t = 0; t < 3; ++t) qf[cb][s].t[t] = as_bf16x8(make_uint4(w[t][0], w[t][1], w[t][2], w[t][3]));
         }
     }
 
@@ -1356,10 +1367,10 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
     const int32_t* table = p.page_table + static_cast<int64_t>(b) * p.pages_per_seq;
     const int64_t head_stride = static_cast<int64_t>(kPageTok) * kDecD;
     const int64_t page_stride = head_stride * p.kv_heads;
-    const uint16_t* kpool = static_cast<const uint16_t*>(p.k_pool) + kvh * head_stride + lr * kDecD + 8 * lg;
-    const uint16_t* vpool = static_cast<const uint16_t*>(p.v_pool) + kvh * head_stride + lr * kPageTok + 4 * lg;
+    const KvT* kpool = static_cast<const KvT*>(p.k_pool) + kvh * head_stride + lr * kDecD + kLane * lg;
+    const KvT* vpool = static_cast<const KvT*>(p.v_pool) + kvh * head_stride + lr * kPageTok + 4 * lg;
     uint4 kb[kKs];
-    uint2 vb[kDt];
+    VecV vb[kDt];
     bool okb = false;
     // page ids 64 at a time, one per lane, so a page's loads wait on no read of
     // their own; an id outside the pool reads page 0 and shows no key
@@ -1373,14 +1384,14 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
         okb = id >= 0 && id < p.num_pages;
         const int64_t base = okb ? static_cast<int64_t>(id) * page_stride : 0;
 #pragma unroll
-        for (int s = 0; s < kKs; ++s) kb[s] = *reinterpret_cast<const uint4*>(kpool + base + 32 * s);
+        for (int s = 0; s < kKs; ++s) kb[s] = *reinterpret_cast<const uint4*>(kpool + base + kStep * s);
 #pragma unroll
-        for (int dt = 0; dt < kDt; ++dt) vb[dt] = *reinterpret_cast<const uint2*>(vpool + base + dt * 16 * kPageTok);
+        for (int dt = 0; dt < kDt; ++dt) vb[dt] = *reinterpret_cast<const VecV*>(vpool + base + dt * 16 * kPageTok);
     };
     if (w_begin < w_end) load_page(w_begin);
     for (int pg = w_begin; pg < w_end; ++pg) {
         uint4 kc[kKs];
-        uint2 vc[kDt];
+        VecV vc[kDt];
 #pragma unroll
         for (int s = 0; s < kKs; ++s) kc[s] = kb[s];
 #pragma unroll
@@ -1394,28 +1405,53 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
             bool bad = false;
 #pragma unroll
             for (int dt = 0; dt < kDt; ++dt) {
-                uint32_t w[2] = {vc[dt].x, vc[dt].y};
+                if constexpr (kF32) {
+                    uint32_t w[4] = {vc[dt].x, vc[dt].y, vc[dt].z, vc[dt].w};
 #pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const uint32_t mask = 0xFFFFu << (16 * (e & 1));
-                    if (!ok || tok0 + e >= len) w[e >> 1] &= ~mask;
-                    const uint32_t expo = (w[e >> 1] >> (16 * (e & 1))) & 0x7F80u;
-                    bad |= expo == 0x7F80u;
+                    for (int e = 0; e < 4; ++e) {
+                        if (!ok || tok0 + e >= len) w[e] = 0u;
+                        bad |= (w[e] & 0x7F800000u) == 0x7F800000u;
+                    }
+                    vc[dt] = make_uint4(w[0], w[1], w[2], w[3]);
+                } else {
+                    uint32_t w[2] = {vc[dt].x, vc[dt].y};
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const uint32_t mask = 0xFFFFu << (16 * (e & 1));
+                        if (!ok || tok0 + e >= len) w[e >> 1] &= ~mask;
+                        const uint32_t expo = (w[e >> 1] >> (16 * (e & 1))) & 0x7F80u;
+                        bad |= expo == 0x7F80u;
+                    }
+                    vc[dt] = make_uint2(w[0], w[1]);
                 }
-                vc[dt] = make_uint2(w[0], w[1]);
             }
             slow = __any(bad);
         }
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) {
-            // three independent chains, the small terms summed first
-            floatx4 st3[3] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+            floatx4 st;
+            if constexpr (kF32) {
+                // two chains; a lane's four dims feed four MFMAs
+                floatx4 s2[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-            for (int s = 0; s < kKs; ++s)
+                for (int s = 0; s < kKs; ++s) {
+                    const float4 kf = __builtin_bit_cast(float4, kc[s]), qq = qf32[cb][s];
+                    s2[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qq.x, s2[0], 0, 0, 0);
+                    s2[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qq.y, s2[1], 0, 0, 0);
+                    s2[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qq.z, s2[0], 0, 0, 0);
+                    s2[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qq.w, s2[1], 0, 0, 0);
+                }
+                st = s2[0] + s2[1];
+            } else {
+                // three independent chains, the small terms summed first
+                floatx4 st3[3] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
-                for (int t = 0; t < 3; ++t)
-                    st3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kc[s]), qf[cb][s].t[t], st3[t], 0, 0, 0);
-            const floatx4 st = st3[0] + (st3[1] + st3[2]);
+                for (int s = 0; s < kKs; ++s)
+#pragma unroll
+                    for (int t = 0; t < 3; ++t)
+                        st3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kc[s]), qf[cb][s].t[t], st3[t], 0, 0, 0);
+                st = st3[0] + (st3[1] + st3[2]);
+            }
             float sv[4];
             float mx = -INFINITY;
 #pragma unroll
@@ -1435,6 +1471,16 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
 #pragma unroll
             for (int dt = 0; dt < kDt; ++dt) acc[cb][dt] *= alpha;
             if (!slow) {
+              if constexpr (kF32) {
+#pragma unroll
+                for (int t = 0; t < 4; ++t)
+#pragma unroll
+                    for (int dt = 0; dt < kDt; ++dt) {
+                        const float4 vf = __builtin_bit_cast(float4, vc[dt]);
+                        const float vt = t == 0 ? vf.x : t == 1 ? vf.y : t == 2 ? vf.z : vf.w;
+                        acc[cb][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vt, pv[t], acc[cb][dt], 0, 0, 0);
+                    }
+              } else {
                 uint16_t w[3][4];
 #pragma unroll
                 for (int r = 0; r < 4; ++r) split3(pv[r], w[0][r], w[1][r], w[2][r]);
@@ -1448,6 +1494,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
 #pragma unroll
                     for (int dt = 0; dt < kDt; ++dt)
                         acc[cb][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as_short4(vc[dt]), pb[t], acc[cb][dt], 0, 0, 0);
+              }
             } else {
                 // token by token: lane (lr, t / 4) holds its probability, lane
                 // (4 lg + r, t / 4) V of this lane's dims
@@ -1458,14 +1505,21 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
                     const bool sees = ok && pg * kPageTok + t < kend[cb];
 #pragma unroll
                     for (int dt = 0; dt < kDt; ++dt) {
-                        // (masked, not selected: a select between the two is turned into a
-                        // load from scratch memory, which would hold V for every page)
+                        // (masked, not selected: a select between the words is turned into
+                        // a load from scratch memory, which would hold V for every page)
                         const uint32_t hi = 0u - static_cast<uint32_t>((t >> 1) & 1);
-                        const uint32_t word = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & hi);
+                        uint32_t word;
+                        if constexpr (kF32) {
+                            const uint32_t odd = 0u - static_cast<uint32_t>(t & 1);
+                            const uint32_t lo2 = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & odd), hi2 = vc[dt].z ^ ((vc[dt].z ^ vc[dt].w) & odd);
+                            word = lo2 ^ ((lo2 ^ hi2) & hi);
+                        } else {
+                            word = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & hi);
+                        }
 #pragma unroll
                         for (int r = 0; r < 4; ++r) {
                             const uint32_t w = __shfl(static_cast<int>(word), 16 * (t >> 2) + 4 * lg + r, 64);
-                            const float v = bf16_to_f32(static_cast<uint16_t>(w >> (16 * (t & 1))));
+                            const float v = kF32 ? __uint_as_float(w) : bf16_to_f32(static_cast<uint16_t>(w >> (16 * (t & 1))));
                             if (sees) acc[cb][dt][r] = fmaf(pt, v, acc[cb][dt][r]);
                         }
                     }
@@ -1587,7 +1641,7 @@ size_t paged_rows_workspace_bytes(int64_t rows, int64_t head_dim, int splits) {
 // The kernel above, where it takes the shape; groups of more than 16 query heads
 // included.  Q is read as 16-byte vectors.
 bool paged_mfma_rows_supported(int kv_dtype, int64_t head_dim, int64_t page_tokens) {
-    return kv_dtype == SFG_BF16 && (head_dim == 128 || head_dim == 64) && page_tokens == kPageTok;
+    return (kv_dtype == SFG_BF16 || kv_dtype == SFG_F32) && (head_dim == 128 || head_dim == 64) && page_tokens == kPageTok;
 }
 
 // Two workgroups per CU (what its registers allow at D = 128) while a split keeps
@@ -1634,9 +1688,9 @@ int launch_attn_paged_rows(const PagedRowsLaunch& a, void* workspace, hipStream_
     p.num_pages = static_cast<int>(a.num_pages); p.splits = a.splits; p.causal = a.causal;
     p.scale = a.scale;
     const dim3 grid(static_cast<unsigned>(rows), static_cast<unsigned>(a.splits));
-    // the matrix-core form reads Q and K as 16-byte vectors and V as 8-byte ones
+    // the matrix-core form reads Q and K as 16-byte vectors and V as 8-byte (fp32: 16-byte) ones
     const bool aligned = ((reinterpret_cast<uintptr_t>(a.q) | reinterpret_cast<uintptr_t>(a.k_pool)) & 15) == 0 &&
-                         (reinterpret_cast<uintptr_t>(a.v_pool) & 7) == 0 && a.q_stride_b % 4 == 0 &&
+                         (reinterpret_cast<uintptr_t>(a.v_pool) & (a.kv_dtype == SFG_F32 ? 15 : 7)) == 0 && a.q_stride_b % 4 == 0 &&
                          a.q_stride_i % 4 == 0 && a.q_stride_h % 4 == 0;
     const int64_t cols = a.seq_q * (a.q_heads / a.kv_heads);
     const int64_t chunks64 = (cols + 15) / 16;
@@ -1644,8 +1698,13 @@ int launch_attn_paged_rows(const PagedRowsLaunch& a, void* workspace, hipStream_
         const int chunks = static_cast<int>(chunks64);
         const dim3 mgrid(static_cast<unsigned>(a.splits), static_cast<unsigned>(a.kv_heads * chunks),
                          static_cast<unsigned>(a.batch));
-        if (a.head_dim == 128) attn_paged_mfma_rows_kernel<128><<<mgrid, 256, 0, stream>>>(p, chunks);
-        else attn_paged_mfma_rows_kernel<64><<<mgrid, 256, 0, stream>>>(p, chunks);
+        if (a.kv_dtype == SFG_F32) {
+            if (a.head_dim == 128) attn_paged_mfma_rows_kernel<float, 128><<<mgrid, 256, 0, stream>>>(p, chunks);
+            else attn_paged_mfma_rows_kernel<float, 64><<<mgrid, 256, 0, stream>>>(p, chunks);
+        } else {
+            if (a.head_dim == 128) attn_paged_mfma_rows_kernel<uint16_t, 128><<<mgrid, 256, 0, stream>>>(p, chunks);
+            else attn_paged_mfma_rows_kernel<uint16_t, 64><<<mgrid, 256, 0, stream>>>(p, chunks);
+        }
     } else if (a.kv_dtype == SFG_F32) attn_paged_rows_kernel<float><<<grid, 64, 0, stream>>>(p);
     else attn_paged_rows_kernel<uint16_t><<<grid, 64, 0, stream>>>(p);
     if (a.mid_event) (void)hipEventRecord(a.mid_event, stream);

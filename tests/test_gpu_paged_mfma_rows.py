@@ -34,16 +34,18 @@ CASES = [(4, 4, 2, 128, 33, 1, 0, False, False), (16, 4, 4, 128, 1000, 1, 0, Fal
          (32, 1, 2, 128, 500, 1, 0, False, True)]
 
 
+@pytest.mark.parametrize("pool", ["bf16", "f32"])
 @pytest.mark.parametrize("hq,hkv,sq,d,longest,causal,splits,unaligned,poison", CASES)
-def test_paged_rows_on_the_matrix_cores(hq, hkv, sq, d, longest, causal, splits, unaligned, poison):
+def test_paged_rows_on_the_matrix_cores(hq, hkv, sq, d, longest, causal, splits, unaligned, poison, pool):
     lib = _abi.load()
     rng = np.random.default_rng(hq * 7 + sq * 3 + longest)
     lens = np.array([longest, 0, 1, max(1, sq - 1), rng.integers(1, longest + 1)], np.int32)
     b, pps = len(lens), (longest + PT - 1) // PT
     pages = b * pps + 3
     table = rng.permutation(pages)[: b * pps].reshape(b, pps).astype(np.int32)
-    kp = oracle.round_bf16(rng.standard_normal((pages, hkv, PT, d)).astype(np.float32))
-    vp = oracle.round_bf16(rng.standard_normal((pages, hkv, d, PT)).astype(np.float32))
+    kp, vp = (rng.standard_normal(s).astype(np.float32) for s in ((pages, hkv, PT, d), (pages, hkv, d, PT)))
+    if pool == "bf16":
+        kp, vp = oracle.round_bf16(kp), oracle.round_bf16(vp)
     q = rng.standard_normal((b, hq, sq, d)).astype(np.float32)
     rows_seen = np.full(b, sq)  # rows compared
     if poison:
@@ -73,13 +75,14 @@ def test_paged_rows_on_the_matrix_cores(hq, hkv, sq, d, longest, causal, splits,
     buf = torch.zeros(q.size + 4, device="cuda")
     qd = buf[1:1 + q.size] if unaligned else buf[:q.size]
     qd.copy_(dev(q).reshape(-1))
-    kd, vd, td, ld = bf16_dev(kp), bf16_dev(vp), dev(table), dev(lens)
+    kv_dtype, to = (F32, dev) if pool == "f32" else (BF16, bf16_dev)
+    kd, vd, td, ld = to(kp), to(vp), dev(table), dev(lens)
     out = torch.zeros((b, hq, sq, d), device="cuda")
-    ws = torch.full((max(1, lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, sq, d, BF16, longest, PT, splits)),), 255,
+    ws = torch.full((max(1, lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, sq, d, kv_dtype, longest, PT, splits)),), 255,
                     dtype=torch.uint8, device="cuda")
     KEEP_ALIVE.extend([buf, out, ws])
     _abi.check(lib.sfg_hip_attn_paged_v1(
-        qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), BF16, td.data_ptr(), ld.data_ptr(), out.data_ptr(), F32, b, hq, hkv,
+        qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), kv_dtype, td.data_ptr(), ld.data_ptr(), out.data_ptr(), F32, b, hq, hkv,
         sq, d, PT, pps, pages, longest, int(causal and sq <= longest), splits, ctypes.c_float(0.0), 0, ws.data_ptr(),
         ws.numel(), stream()))
     torch.cuda.synchronize()
