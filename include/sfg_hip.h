@@ -302,8 +302,8 @@ int sfg_hip_attn_decode_paged_noalloc_v1(const float* q, const uint16_t* k_pool,
  * so seq_q = 1 sees all of them.  A row with no visible key comes out NaN, as
  * the reference's 0 / 0.  The MFMA split kernel takes the shapes it lowers
  * (bf16, head_dim 64 / 128, 16-token pages, one row, GQA group up to 16);
- * other bf16 shapes with that head_dim and page size run an MFMA kernel that
- * keeps Q and the probabilities at fp32 precision; the rest one wave per
+ * other shapes with that head_dim and page size, fp32 pools among them, run an
+ * MFMA kernel that keeps Q and the probabilities at fp32 precision; the rest one wave per
  * (sequence, row, head, split) with fp32 dot products over the head dimension
  * and an fp32 online softmax.  Errors:
  * SFG_ERR_INVALID_CONFIG for causal with seq_q > max_context (validate_config,
