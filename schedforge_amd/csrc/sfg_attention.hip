@@ -1254,16 +1254,26 @@ __global__ __launch_bounds__(64) void attn_paged_rows_kernel(PagedRowsArgs p) {
 //
 // A page holding keys hidden from some rows or past the sequence's end zeroes V
 // past the end, and takes its tokens one at a time if a hidden one is not
-// finite (0 * inf).
+// finite (0 * inf).  Bf16 pools: an infinite key or value that a row does see
+// meets the three terms one by one, which gives NaN (0 * inf, inf - inf) where
+// the product of the whole value is infinite.  So a wave whose sums are not
+// finite at the end walks its pages once more: keys' non-finite elements meet
+// the leading term only, and pages with a non-finite value go token by token.
 // ===========================================================================
 struct Bf16x3 {
     bf16x8 t[3];
 };
+// (truncated terms: a rounded leading one could overflow to infinity)
 __device__ __forceinline__ void split3(float v, uint16_t& hi, uint16_t& mid, uint16_t& lo) {
-    hi = f32_to_bf16(v);
+    hi = static_cast<uint16_t>(__float_as_uint(v) >> 16);
     const float r = v - bf16_to_f32(hi);
-    mid = f32_to_bf16(r);
-    lo = f32_to_bf16(r - bf16_to_f32(mid));
+    mid = static_cast<uint16_t>(__float_as_uint(r) >> 16);
+    lo = static_cast<uint16_t>(__float_as_uint(r - bf16_to_f32(mid)) >> 16);
+}
+// two bf16 values, the infinite and NaN ones replaced by zero
+__device__ __forceinline__ uint32_t finite_bf16x2(uint32_t w) {
+    const uint32_t bad = ((w & 0x7F807F80u) + 0x00800080u) & 0x80008000u;  // exponent all ones
+    return w & ~((bad >> 15) * 0xFFFFu);
 }
 
 template <typename KvT, int kDecD>
@@ -1357,13 +1367,6 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
 
     floatx4 acc[NCB][kDt];
     float m_run[NCB], l_run[NCB];
-#pragma unroll
-    for (int cb = 0; cb < NCB; ++cb) {
-        m_run[cb] = -INFINITY;
-        l_run[cb] = 0.f;
-#pragma unroll
-        for (int i = 0; i < kDt; ++i) acc[cb][i] = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
     const int32_t* table = p.page_table + static_cast<int64_t>(b) * p.pages_per_seq;
     const int64_t head_stride = static_cast<int64_t>(kPageTok) * kDecD;
     const int64_t page_stride = head_stride * p.kv_heads;
@@ -1388,144 +1391,175 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
 #pragma unroll
         for (int dt = 0; dt < kDt; ++dt) vb[dt] = *reinterpret_cast<const VecV*>(vpool + base + dt * 16 * kPageTok);
     };
-    if (w_begin < w_end) load_page(w_begin);
-    for (int pg = w_begin; pg < w_end; ++pg) {
-        uint4 kc[kKs];
-        VecV vc[kDt];
-#pragma unroll
-        for (int s = 0; s < kKs; ++s) kc[s] = kb[s];
-#pragma unroll
-        for (int dt = 0; dt < kDt; ++dt) vc[dt] = vb[dt];
-        const bool ok = okb;
-        if (pg + 1 < w_end) load_page(pg + 1);
-        const int tok0 = pg * kPageTok + 4 * lg;  // this lane's four tokens
-        bool slow = false;
-        if (!ok || (pg + 1) * kPageTok > all_see) {  // wave-uniform
-            // tokens past the end (or of no page) are not data
-            bool bad = false;
-#pragma unroll
-            for (int dt = 0; dt < kDt; ++dt) {
-                if constexpr (kF32) {
-                    uint32_t w[4] = {vc[dt].x, vc[dt].y, vc[dt].z, vc[dt].w};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        if (!ok || tok0 + e >= len) w[e] = 0u;
-                        bad |= (w[e] & 0x7F800000u) == 0x7F800000u;
-                    }
-                    vc[dt] = make_uint4(w[0], w[1], w[2], w[3]);
-                } else {
-                    uint32_t w[2] = {vc[dt].x, vc[dt].y};
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const uint32_t mask = 0xFFFFu << (16 * (e & 1));
-                        if (!ok || tok0 + e >= len) w[e >> 1] &= ~mask;
-                        const uint32_t expo = (w[e >> 1] >> (16 * (e & 1))) & 0x7F80u;
-                        bad |= expo == 0x7F80u;
-                    }
-                    vc[dt] = make_uint2(w[0], w[1]);
-                }
-            }
-            slow = __any(bad);
-        }
+    // the second walk is for bf16 pools with visible non-finite elements
+    for (int walk = 0;; ++walk) {
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) {
-            floatx4 st;
-            if constexpr (kF32) {
-                // two chains; a lane's four dims feed four MFMAs
-                floatx4 s2[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+            m_run[cb] = -INFINITY;
+            l_run[cb] = 0.f;
 #pragma unroll
-                for (int s = 0; s < kKs; ++s) {
-                    const float4 kf = __builtin_bit_cast(float4, kc[s]), qq = qf32[cb][s];
-                    s2[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qq.x, s2[0], 0, 0, 0);
-                    s2[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qq.y, s2[1], 0, 0, 0);
-                    s2[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qq.z, s2[0], 0, 0, 0);
-                    s2[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qq.w, s2[1], 0, 0, 0);
+            for (int i = 0; i < kDt; ++i) acc[cb][i] = floatx4{0.f, 0.f, 0.f, 0.f};
+        }
+        ids_base = w_begin - 64;
+        if (w_begin < w_end) load_page(w_begin);
+        for (int pg = w_begin; pg < w_end; ++pg) {
+            uint4 kc[kKs];
+            VecV vc[kDt];
+#pragma unroll
+            for (int s = 0; s < kKs; ++s) kc[s] = kb[s];
+#pragma unroll
+            for (int dt = 0; dt < kDt; ++dt) vc[dt] = vb[dt];
+            const bool ok = okb;
+            if (pg + 1 < w_end) load_page(pg + 1);
+            const int tok0 = pg * kPageTok + 4 * lg;  // this lane's four tokens
+            bool slow = false;
+            if (!ok || walk > 0 || (pg + 1) * kPageTok > all_see) {  // wave-uniform
+                // tokens past the end (or of no page) are not data
+                bool bad = false;
+#pragma unroll
+                for (int dt = 0; dt < kDt; ++dt) {
+                    if constexpr (kF32) {
+                        uint32_t w[4] = {vc[dt].x, vc[dt].y, vc[dt].z, vc[dt].w};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            if (!ok || tok0 + e >= len) w[e] = 0u;
+                            bad |= (w[e] & 0x7F800000u) == 0x7F800000u;
+                        }
+                        vc[dt] = make_uint4(w[0], w[1], w[2], w[3]);
+                    } else {
+                        uint32_t w[2] = {vc[dt].x, vc[dt].y};
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const uint32_t mask = 0xFFFFu << (16 * (e & 1));
+                            if (!ok || tok0 + e >= len) w[e >> 1] &= ~mask;
+                            const uint32_t expo = (w[e >> 1] >> (16 * (e & 1))) & 0x7F80u;
+                            bad |= expo == 0x7F80u;
+                        }
+                        vc[dt] = make_uint2(w[0], w[1]);
+                    }
                 }
-                st = s2[0] + s2[1];
-            } else {
-                // three independent chains, the small terms summed first
-                floatx4 st3[3] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+                slow = __any(bad);
+            }
 #pragma unroll
-                for (int s = 0; s < kKs; ++s)
+            for (int cb = 0; cb < NCB; ++cb) {
+                floatx4 st;
+                if constexpr (kF32) {
+                    // two chains; a lane's four dims feed four MFMAs
+                    floatx4 s2[2] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+                    for (int s = 0; s < kKs; ++s) {
+                        const float4 kf = __builtin_bit_cast(float4, kc[s]), qq = qf32[cb][s];
+                        s2[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.x, qq.x, s2[0], 0, 0, 0);
+                        s2[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.y, qq.y, s2[1], 0, 0, 0);
+                        s2[0] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.z, qq.z, s2[0], 0, 0, 0);
+                        s2[1] = __builtin_amdgcn_mfma_f32_16x16x4f32(kf.w, qq.w, s2[1], 0, 0, 0);
+                    }
+                    st = s2[0] + s2[1];
+                } else {
+                    // three independent chains, the small terms summed first
+                    floatx4 st3[3] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
+                    auto scores = [&](auto finite_c) __attribute__((always_inline)) {
+#pragma unroll
+                        for (int s = 0; s < kKs; ++s)
+#pragma unroll
+                            for (int t = 0; t < 3; ++t) {
+                                uint4 k = kc[s];
+                                if (decltype(finite_c)::value && t > 0)
+                                    k = make_uint4(finite_bf16x2(k.x), finite_bf16x2(k.y), finite_bf16x2(k.z), finite_bf16x2(k.w));
+                                st3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), qf[cb][s].t[t], st3[t], 0, 0, 0);
+                            }
+                    };
+                    if (walk == 0) scores(std::false_type{});
+                    else scores(std::true_type{});
+                    st = st3[0] + (st3[1] + st3[2]);
+                }
+                float sv[4];
+                float mx = -INFINITY;
+#pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    sv[r] = ok && tok0 + r < kend[cb] ? st[r] * p.scale : -INFINITY;
+                    mx = fmaxf(mx, sv[r]);
+                }
+                mx = xor16_max(mx);
+                mx = xor32_max(mx);
+                const float m_new = fmaxf(m_run[cb], mx);
+                const float alpha = m_run[cb] == -INFINITY ? 0.f : expf(m_run[cb] - m_new);
+                float pv[4];
+#pragma unroll
+                for (int r = 0; r < 4; ++r) pv[r] = sv[r] == -INFINITY ? 0.f : expf(sv[r] - m_new);
+                l_run[cb] = l_run[cb] * alpha + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
+                m_run[cb] = m_new;
+#pragma unroll
+                for (int dt = 0; dt < kDt; ++dt) acc[cb][dt] *= alpha;
+                if (!slow) {
+                  if constexpr (kF32) {
+#pragma unroll
+                    for (int t = 0; t < 4; ++t)
+#pragma unroll
+                        for (int dt = 0; dt < kDt; ++dt) {
+                            const float4 vf = __builtin_bit_cast(float4, vc[dt]);
+                            const float vt = t == 0 ? vf.x : t == 1 ? vf.y : t == 2 ? vf.z : vf.w;
+                            acc[cb][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vt, pv[t], acc[cb][dt], 0, 0, 0);
+                        }
+                  } else {
+                    uint16_t w[3][4];
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) split3(pv[r], w[0][r], w[1][r], w[2][r]);
+                    short4v pb[3];
 #pragma unroll
                     for (int t = 0; t < 3; ++t)
-                        st3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(kc[s]), qf[cb][s].t[t], st3[t], 0, 0, 0);
-                st = st3[0] + (st3[1] + st3[2]);
-            }
-            float sv[4];
-            float mx = -INFINITY;
+                        pb[t] = as_short4(make_uint2(static_cast<uint32_t>(w[t][0]) | (static_cast<uint32_t>(w[t][1]) << 16),
+                                                     static_cast<uint32_t>(w[t][2]) | (static_cast<uint32_t>(w[t][3]) << 16)));
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                sv[r] = ok && tok0 + r < kend[cb] ? st[r] * p.scale : -INFINITY;
-                mx = fmaxf(mx, sv[r]);
-            }
-            mx = xor16_max(mx);
-            mx = xor32_max(mx);
-            const float m_new = fmaxf(m_run[cb], mx);
-            const float alpha = m_run[cb] == -INFINITY ? 0.f : expf(m_run[cb] - m_new);
-            float pv[4];
+                    for (int t = 2; t >= 0; --t)
 #pragma unroll
-            for (int r = 0; r < 4; ++r) pv[r] = sv[r] == -INFINITY ? 0.f : expf(sv[r] - m_new);
-            l_run[cb] = l_run[cb] * alpha + ((pv[0] + pv[1]) + (pv[2] + pv[3]));
-            m_run[cb] = m_new;
-#pragma unroll
-            for (int dt = 0; dt < kDt; ++dt) acc[cb][dt] *= alpha;
-            if (!slow) {
-              if constexpr (kF32) {
-#pragma unroll
-                for (int t = 0; t < 4; ++t)
-#pragma unroll
-                    for (int dt = 0; dt < kDt; ++dt) {
-                        const float4 vf = __builtin_bit_cast(float4, vc[dt]);
-                        const float vt = t == 0 ? vf.x : t == 1 ? vf.y : t == 2 ? vf.z : vf.w;
-                        acc[cb][dt] = __builtin_amdgcn_mfma_f32_16x16x4f32(vt, pv[t], acc[cb][dt], 0, 0, 0);
-                    }
-              } else {
-                uint16_t w[3][4];
-#pragma unroll
-                for (int r = 0; r < 4; ++r) split3(pv[r], w[0][r], w[1][r], w[2][r]);
-                short4v pb[3];
-#pragma unroll
-                for (int t = 0; t < 3; ++t)
-                    pb[t] = as_short4(make_uint2(static_cast<uint32_t>(w[t][0]) | (static_cast<uint32_t>(w[t][1]) << 16),
-                                                 static_cast<uint32_t>(w[t][2]) | (static_cast<uint32_t>(w[t][3]) << 16)));
-#pragma unroll
-                for (int t = 2; t >= 0; --t)
-#pragma unroll
-                    for (int dt = 0; dt < kDt; ++dt)
-                        acc[cb][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as_short4(vc[dt]), pb[t], acc[cb][dt], 0, 0, 0);
-              }
-            } else {
-                // token by token: lane (lr, t / 4) holds its probability, lane
-                // (4 lg + r, t / 4) V of this lane's dims
+                        for (int dt = 0; dt < kDt; ++dt)
+                            acc[cb][dt] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(as_short4(vc[dt]), pb[t], acc[cb][dt], 0, 0, 0);
+                  }
+                } else {
+                    // token by token: lane (lr, t / 4) holds its probability, lane
+                    // (4 lg + r, t / 4) V of this lane's dims
 #pragma unroll 1
-                for (int t = 0; t < kPageTok; ++t) {
-                    const float mine = (t & 3) == 0 ? pv[0] : (t & 3) == 1 ? pv[1] : (t & 3) == 2 ? pv[2] : pv[3];
-                    const float pt = __shfl(mine, 16 * (t >> 2) + lr, 64);
-                    const bool sees = ok && pg * kPageTok + t < kend[cb];
+                    for (int t = 0; t < kPageTok; ++t) {
+                        const float mine = (t & 3) == 0 ? pv[0] : (t & 3) == 1 ? pv[1] : (t & 3) == 2 ? pv[2] : pv[3];
+                        const float pt = __shfl(mine, 16 * (t >> 2) + lr, 64);
+                        const bool sees = ok && pg * kPageTok + t < kend[cb];
 #pragma unroll
-                    for (int dt = 0; dt < kDt; ++dt) {
-                        // (masked, not selected: a select between the words is turned into
-                        // a load from scratch memory, which would hold V for every page)
-                        const uint32_t hi = 0u - static_cast<uint32_t>((t >> 1) & 1);
-                        uint32_t word;
-                        if constexpr (kF32) {
-                            const uint32_t odd = 0u - static_cast<uint32_t>(t & 1);
-                            const uint32_t lo2 = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & odd), hi2 = vc[dt].z ^ ((vc[dt].z ^ vc[dt].w) & odd);
-                            word = lo2 ^ ((lo2 ^ hi2) & hi);
-                        } else {
-                            word = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & hi);
-                        }
+                        for (int dt = 0; dt < kDt; ++dt) {
+                            // (masked, not selected: a select between the words is turned into
+                            // a load from scratch memory, which would hold V for every page)
+                            const uint32_t hi = 0u - static_cast<uint32_t>((t >> 1) & 1);
+                            uint32_t word;
+                            if constexpr (kF32) {
+                                const uint32_t odd = 0u - static_cast<uint32_t>(t & 1);
+                                const uint32_t lo2 = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & odd), hi2 = vc[dt].z ^ ((vc[dt].z ^ vc[dt].w) & odd);
+                                word = lo2 ^ ((lo2 ^ hi2) & hi);
+                            } else {
+                                word = vc[dt].x ^ ((vc[dt].x ^ vc[dt].y) & hi);
+                            }
 #pragma unroll
-                        for (int r = 0; r < 4; ++r) {
-                            const uint32_t w = __shfl(static_cast<int>(word), 16 * (t >> 2) + 4 * lg + r, 64);
-                            const float v = kF32 ? __uint_as_float(w) : bf16_to_f32(static_cast<uint16_t>(w >> (16 * (t & 1))));
-                            if (sees) acc[cb][dt][r] = fmaf(pt, v, acc[cb][dt][r]);
+                            for (int r = 0; r < 4; ++r) {
+                                const uint32_t w = __shfl(static_cast<int>(word), 16 * (t >> 2) + 4 * lg + r, 64);
+                                const float v = kF32 ? __uint_as_float(w) : bf16_to_f32(static_cast<uint16_t>(w >> (16 * (t & 1))));
+                                if (sees) acc[cb][dt][r] = fmaf(pt, v, acc[cb][dt][r]);
+                            }
                         }
                     }
                 }
             }
         }
+        if (kF32 || walk > 0) break;
+        bool bad = false;
+#pragma unroll
+        for (int cb = 0; cb < NCB; ++cb) {
+            float t = l_run[cb] * 0.f;  // NaN unless every sum is finite
+#pragma unroll
+            for (int dt = 0; dt < kDt; ++dt)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) t = fmaf(acc[cb][dt][r], 0.f, t);
+            bad |= kend[cb] > 0 && t != 0.f;
+        }
+        if (!__any(bad)) break;
     }
     // merge the four waves in LDS: acc[cb][dt][r] = O^T[dim 16 dt + 4 lg + r][column lr]
     constexpr int kCols = 16 * NCB;

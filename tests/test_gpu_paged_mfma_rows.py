@@ -95,6 +95,91 @@ def test_paged_rows_on_the_matrix_cores(hq, hkv, sq, d, longest, causal, splits,
             assert err < 3e-6, (n, err)
 
 
+def _reference(q, kp, vp, table, lens, causal):
+    """softmax(q k / sqrt(d)) v in float64, infinities and NaN as they come."""
+    b, hq, sq, d = q.shape
+    hkv = kp.shape[1]
+    ref = np.full(q.shape, np.nan)
+    with np.errstate(invalid="ignore", over="ignore"):
+        for n in range(b):
+            L = int(lens[n])
+            k = kp[table[n]].transpose(1, 0, 2, 3).reshape(hkv, -1, d)[:, :L].astype(np.float64)
+            v = vp[table[n]].transpose(1, 0, 3, 2).reshape(hkv, -1, d)[:, :L].astype(np.float64)
+            for h in range(hq):
+                j = h * hkv // hq
+                for i in range(sq):
+                    end = min(L, L - sq + i + 1) if causal else L
+                    s = (k[j, :end] * q[n, h, i].astype(np.float64)).sum(axis=1) / np.sqrt(d)
+                    p = np.exp(s - s.max())
+                    ref[n, h, i] = ((p / p.sum())[:, None] * v[j, :end]).sum(axis=0)
+    return ref
+
+
+def _run_paged(q, kp, vp, table, lens, causal, splits, pool):
+    lib = _abi.load()
+    b, hq, sq, d = q.shape
+    pages, hkv = kp.shape[:2]
+    longest, pps = int(lens.max()), table.shape[1]
+    kv_dtype, to = (F32, dev) if pool == "f32" else (BF16, bf16_dev)
+    qd, kd, vd, td, ld = dev(q), to(kp), to(vp), dev(table), dev(lens)
+    out = torch.zeros(q.shape, device="cuda")
+    n = lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, sq, d, kv_dtype, longest, PT, splits)
+    ws = torch.full((max(1, n),), 255, dtype=torch.uint8, device="cuda")
+    KEEP_ALIVE.extend([out, ws])
+    _abi.check(lib.sfg_hip_attn_paged_v1(
+        qd.data_ptr(), kd.data_ptr(), vd.data_ptr(), kv_dtype, td.data_ptr(), ld.data_ptr(), out.data_ptr(), F32, b, hq, hkv,
+        sq, d, PT, pps, pages, longest, causal, splits, ctypes.c_float(0.0), 0, ws.data_ptr(), ws.numel(), stream()))
+    torch.cuda.synchronize()
+    return host(out)
+
+
+def _check_non_finite(got, ref):
+    np.testing.assert_array_equal(np.isnan(got), np.isnan(ref))
+    inf = np.isinf(ref)
+    np.testing.assert_array_equal(got[inf], ref[inf])
+    fin = np.isfinite(ref)
+    assert np.isfinite(got[fin]).all()
+    assert np.abs(got[fin] - ref[fin]).max() < 3e-6 * np.abs(ref[fin]).max()
+
+
+def _random_pools(rng, b, hq, hkv, sq, d, longest, pool):
+    pps = (longest + PT - 1) // PT
+    table = rng.permutation(b * pps).reshape(b, pps).astype(np.int32)
+    kp, vp = (rng.standard_normal(s).astype(np.float32) for s in ((b * pps, hkv, PT, d), (b * pps, hkv, d, PT)))
+    if pool == "bf16":
+        kp, vp = oracle.round_bf16(kp), oracle.round_bf16(vp)
+    return table, kp, vp, rng.standard_normal((b, hq, sq, d)).astype(np.float32)
+
+
+# sequence 0: keys of -inf against positive query elements (exact in bf16 and not),
+# weight 0; 1: infinite values; 2: both, on every page; 3: a key of +inf, so NaN;
+# 4: a query element above the largest bf16 against tiny key elements
+@pytest.mark.parametrize("pool", ["bf16", "f32"])
+@pytest.mark.parametrize("hq,hkv,sq,d,longest,causal,splits", [(16, 4, 2, 128, 300, 1, 0), (8, 2, 5, 64, 70, 1, 1),
+                                                               (12, 2, 3, 128, 130, 0, 3), (34, 2, 1, 64, 200, 1, 0)])
+def test_visible_infinities_give_the_reference_result(hq, hkv, sq, d, longest, causal, splits, pool):
+    rng = np.random.default_rng(d + longest)
+    b = 5
+    table, kp, vp, q = _random_pools(rng, b, hq, hkv, sq, d, longest, pool)
+    lens = np.array([longest, longest - 1, longest, longest - 3, longest], np.int32)
+    q[..., 3] = 1.0
+    q[..., 9] = np.abs(q[..., 9]) + 0.1
+    q[4, ..., 5] = 3.4e38
+    for n, keys, values in ((0, 0, None), (1, None, 0), (2, 0, 3)):
+        for t in range(0, lens[n] - sq - 3, 7):  # tokens that every row sees
+            if keys is not None:
+                kp[table[n, t // PT], :, t % PT, 3 if t % 2 else 9] = -np.inf
+            if values is not None:
+                pg, at = table[n, (t + values) // PT], (t + values) % PT
+                vp[pg, :, 1::5, at] = np.inf
+                vp[pg, :, 2::5, at] = -np.inf
+    kp[table[3, 1], :, 4, 9] = np.inf
+    kp[table[4], ..., 5] = np.copysign(np.float32(2.0 ** -125), kp[table[4], ..., 5])
+    ref = _reference(q, kp, vp, table, lens, causal)
+    assert np.isfinite(ref[0]).all() and np.isinf(ref[1]).any() and np.isnan(ref[3]).all() and np.isfinite(ref[4]).all()
+    _check_non_finite(_run_paged(q, kp, vp, table, lens, causal, splits, pool), ref)
+
+
 def test_decode_workspace_covers_every_kv_head_count():
     """The one-row workspace query, which is not told the kv head count."""
     lib = _abi.load()
