@@ -1802,6 +1802,14 @@ bool fits_32bit(int64_t a_rows, int64_t lda, int a_elem, int64_t b_rows, int64_t
     return static_cast<uint64_t>(a_rows) * lda * a_elem + slack <= 0xFFFFFFFFull &&
            static_cast<uint64_t>(b_rows) * ldb * b_elem + slack <= 0xFFFFFFFFull;
 }
+
+// Every bf16 / int8 MFMA kernel reads A and B rows as 16-byte vectors and steps
+// k by 32: other rows and depths run on the VALU kernel.
+bool mfma_operands(const GemmProblem& p) {
+    const int64_t b_elem = p.b_dtype == SFG_I8 ? 1 : 2;
+    return ((reinterpret_cast<uintptr_t>(p.a) | reinterpret_cast<uintptr_t>(p.b)) & 15) == 0 &&
+           (p.lda * 2) % 16 == 0 && (p.ldb * b_elem) % 16 == 0 && p.k % kTK == 0;
+}
 }  // namespace
 
 // The tile launch_gemm gives a product on the ring / 256 x 256 kernels.
@@ -1815,7 +1823,7 @@ RingPlan tile_plan(const GemmProblem& p, bool glu, int groups, bool split, size_
 bool gemm_qkv_rope_supported(const GemmProblem& p) {
     const QkvRopeOut& o = p.qkv;
     if (!(p.a_dtype == SFG_BF16 && (p.b_dtype == SFG_BF16 || (p.b_dtype == SFG_I8 && p.b_scales)) && !p.offsets &&
-          !p.a_rows && p.b_layout == SFG_LAYOUT_NK && p.m > kSkinnyMaxRows && p.k % kTK == 0 && o.rope && o.q && o.k &&
+          !p.a_rows && p.b_layout == SFG_LAYOUT_NK && p.m > kSkinnyMaxRows && mfma_operands(p) && o.rope && o.q && o.k &&
           o.vt && o.seq >= 4 && p.m % o.seq == 0 && o.q_heads > 0 && o.kv_heads > 0 &&
           p.n == (static_cast<int64_t>(o.q_heads) + 2 * o.kv_heads) * 128 && o.ld_vt % 64 == 0 && o.ld_vt >= o.seq &&
           fits_32bit(p.m, p.lda, 2, p.n, p.ldb, p.b_dtype == SFG_I8 ? 1 : 2, p.k)))
@@ -1873,12 +1881,7 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
     if (p.a_dtype != SFG_BF16 || (p.b_dtype != SFG_BF16 && p.b_dtype != SFG_I8))
         return SFG_ERR_UNSUPPORTED;
     if (p.b_dtype == SFG_I8 && p.b_scales == nullptr) return SFG_ERR_SHAPE;
-    // every bf16 / int8 MFMA kernel reads A and B rows as 16-byte vectors and
-    // steps k by 32: other rows and depths run on the VALU kernel
-    const int64_t b_elem = p.b_dtype == SFG_I8 ? 1 : 2;
-    if ((reinterpret_cast<uintptr_t>(p.a) & 15) || (reinterpret_cast<uintptr_t>(p.b) & 15) ||
-        (p.lda * 2) % 16 != 0 || (p.ldb * b_elem) % 16 != 0 || p.k % kTK != 0)
-        return launch_vec(p, stream);
+    if (!mfma_operands(p)) return launch_vec(p, stream);
     const int groups = p.offsets ? p.groups : 1;
     // 33..64 dense rows: split-K slices when the caller's workspace holds the
     // partial sums (sized by gemm_workspace_bytes).

@@ -103,3 +103,25 @@ def test_qkv_epilogue_on_ragged_sequences(dtype, batch, seq):
     if dtype == "bf16":  # the same bits as a tile named by the plan
         plan.desc.gemm_tile = _abi.TILE_128x128
         assert np.array_equal(execute_decoder_layer(plan, d.input, warmup=0, repetitions=1).output, out)
+
+
+# weights that do not start on 16 bytes: the fused epilogue's tiles read whole
+# 16-byte vectors, so such a layer takes the separate split + RoPE pass
+@pytest.mark.parametrize("dtype,batch,seq", [("bf16", 2, 40), ("bf16", 4, 257), ("w8", 2, 40)])
+def test_prefill_layer_with_unaligned_qkv_weights(dtype, batch, seq):
+    import oracle
+    from schedforge_amd import CONFIGS
+    from schedforge_amd.layer import compile_decoder, execute_decoder_layer
+    from _helpers import TOL, decoder_data
+    cfg = CONFIGS["c4"].replace(batch=batch, sequence=seq, hidden=512, intermediate=512, query_heads=4, kv_heads=2,
+                                dtype=dtype)
+    d = oracle.make_layer_data(cfg, 4300 + seq)
+    plan = compile_decoder(cfg, decoder_data(d), "cuda")
+    w = plan.t["w_qkv"].reshape(-1)
+    off = 1 if dtype == "bf16" else 2  # elements: 2 bytes either way
+    moved = torch.empty(w.numel() + 16, dtype=w.dtype, device="cuda")
+    moved[off:off + w.numel()] = w
+    KEEP_ALIVE.append(moved)
+    plan.weights.w_qkv = moved.data_ptr() + 2
+    out = execute_decoder_layer(plan, d.input, warmup=0, repetitions=1).output
+    assert oracle.rel_error(out, oracle.decoder_layer(cfg, d)) < TOL[dtype]
