@@ -192,7 +192,15 @@ int launch_attn_prefill_f32(const float* q, const float* k, const float* v, void
                             int64_t seq_q, int64_t seq_kv, int64_t head_dim, int causal,
                             float scale, hipStream_t stream) {
     if (head_dim > kRowMaxD) return SFG_ERR_UNSUPPORTED;
-    if (attn_prefill_f32_mfma_supported(q, k, v, out, batch, q_heads, seq_q, seq_kv, head_dim))
+    // The row kernel holds 64 keys in LDS and takes four rows a workgroup, one
+    // workgroup a CU: a few short rounds of it end before one of the flash kernel's
+    // 32-row blocks.  6000 seeded calls: 8 rows x 8 keys 4.4 us against 9.1 (D 64),
+    // 12.7 (D 128); they meet at 68 and 150 keys in one round (48 - 63 keys 0.84 x the
+    // flash kernel's time at D 64, 80 - 95 1.18 x), at 20 and 22 in two.  (At D 64 the
+    // line is 60 keys: prompts of 64 and of 128 tokens give shared rows the same bits.)
+    const int64_t rounds = (batch * q_heads * ((seq_q + 3) / 4) + 255) / 256;
+    const bool rows_faster = head_dim == 64 ? rounds * (seq_kv + 28) <= 88 : rounds * (seq_kv + 106) <= 256;
+    if (!rows_faster && attn_prefill_f32_mfma_supported(q, k, v, out, batch, q_heads, seq_q, seq_kv, head_dim))
         launch_attn_prefill_f32_mfma(q, k, v, out, out_dtype, batch, q_heads, kv_heads, seq_q, seq_kv, head_dim,
                                      causal, scale, stream);
     else

@@ -291,13 +291,13 @@ void launch_f32_flash(const float* q, const float* k, const float* v, void* out,
 }  // namespace
 
 // head_dim 64 / 128, 16-byte aligned tensors, K and V of one head within 32-bit
-// byte offsets, a grid within 31 bits.
+// byte offsets, a grid within 32 bits of work items.
 bool attn_prefill_f32_mfma_supported(const float* q, const float* k, const float* v, const void* out,
                                      int64_t batch, int64_t q_heads, int64_t seq_q, int64_t seq_kv, int64_t head_dim) {
     const uintptr_t low = reinterpret_cast<uintptr_t>(q) | reinterpret_cast<uintptr_t>(k) |
                           reinterpret_cast<uintptr_t>(v) | reinterpret_cast<uintptr_t>(out);
     return (head_dim == 64 || head_dim == 128) && (low & 15) == 0 && seq_kv <= (int64_t(1) << 22) &&
-           seq_q <= (int64_t(1) << 22) && batch * q_heads * ((seq_q + 31) / 32) < (int64_t(1) << 31);
+           seq_q <= (int64_t(1) << 22) && batch * q_heads * ((seq_q + 31) / 32) < (int64_t(1) << 24);
 }
 
 void launch_attn_prefill_f32_mfma(const float* q, const float* k, const float* v, void* out, int out_dtype,

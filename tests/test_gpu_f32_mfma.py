@@ -107,3 +107,15 @@ def test_f32_flash_prefill(b, hq, hkv, sq, skv, d, causal, poison):
         got = (host(out) if out_dtype == F32 else bf16_host(out))[:, :rows]
         err = np.abs(got - ref[:, :rows]).max(initial=0.0) / max(np.abs(ref[:, :rows]).max(initial=0.0), 1e-6)
         assert err < (2e-6 if out_dtype == F32 else 4e-3), (err, out_dtype)
+
+
+# either side of the line to the row kernel: keys of one round of workgroups (60 and
+# 150), one round and two (blocks of four rows over 256), short keys in many rounds
+@pytest.mark.parametrize("b,hq,hkv,sq,skv,d,causal", [
+    (1, 2, 1, 60, 60, 64, 1), (1, 2, 1, 61, 61, 64, 1), (2, 2, 2, 150, 150, 128, 1), (2, 2, 1, 151, 151, 128, 0),
+    (8, 8, 4, 16, 16, 64, 1), (8, 8, 2, 17, 33, 64, 1), (16, 8, 8, 22, 22, 128, 1), (16, 8, 2, 9, 23, 128, 1),
+    (40, 16, 4, 1, 1, 64, 1), (40, 16, 4, 5, 7, 128, 0)])
+def test_f32_prefill_at_the_row_kernels_line(b, hq, hkv, sq, skv, d, causal):
+    test_f32_flash_prefill(b, hq, hkv, sq, skv, d, causal, False)
+    if causal:
+        test_f32_flash_prefill(b, hq, hkv, sq, skv, d, causal, True)
