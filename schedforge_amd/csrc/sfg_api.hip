@@ -75,6 +75,7 @@ int check_decode_args(const float* q, const void* k_pool, const void* v_pool,
 // head_dim <= 256, page size, new-token count and pool dtype), in its
 // matrix-core form (rows_mfma) where that takes the shape.  `bytes` is the
 // partials' workspace; both forms of the row kernel leave the same partials.
+// ragged: the sequences have lengths of their own (never fewer splits than without).
 struct DecodePlan {
     bool mfma;
     int splits;
@@ -83,9 +84,10 @@ struct DecodePlan {
 };
 
 DecodePlan plan_decode(int kv_dtype, int64_t batch, int64_t q_heads, int64_t kv_heads, int64_t seq_q,
-                       int64_t head_dim, int64_t page_tokens, int64_t max_context, int32_t kv_splits) {
+                       int64_t head_dim, int64_t page_tokens, int64_t max_context, int32_t kv_splits,
+                       bool ragged = true) {
     if (sfg::decode_mfma_supported(kv_dtype, head_dim, page_tokens, q_heads / kv_heads, seq_q)) {
-        const int s = sfg::decode_split_count(batch, kv_heads, max_context, page_tokens, kv_splits);
+        const int s = sfg::decode_split_count(batch, kv_heads, head_dim, max_context, page_tokens, kv_splits, ragged);
         return {true, s, sfg::decode_workspace_bytes(batch, q_heads, head_dim, s)};
     }
     const int64_t rows = batch * seq_q * q_heads;
@@ -527,7 +529,7 @@ size_t sfg_hip_attn_decode_workspace_v1(int64_t batch, int64_t q_heads, int64_t 
     // for any kv_heads.  The row kernel's partials (shapes the MFMA kernel does
     // not lower) are covered too.
     if (batch <= 0 || q_heads <= 0 || head_dim <= 0 || max_context <= 0 || page_tokens <= 0) return 0;
-    const int s = sfg::decode_split_count(batch, 1, max_context, page_tokens, kv_splits);
+    const int s = sfg::decode_split_count(batch, 1, head_dim, max_context, page_tokens, kv_splits, true);
     const size_t mfma = sfg::decode_workspace_bytes(batch, q_heads, head_dim, s);
     const int rs = sfg::paged_rows_split_count(batch * q_heads, max_context, kv_splits);
     size_t rows = sfg::paged_rows_workspace_bytes(batch * q_heads, head_dim, rs);
@@ -553,7 +555,7 @@ int sfg_hip_attn_decode_paged_v1(const float* q, const uint16_t* k_pool, const u
                                 stream)) != SFG_OK)
         return rc;
     const DecodePlan plan = plan_decode(SFG_BF16, batch, q_heads, kv_heads, 1, head_dim, page_tokens,
-                                        max_context, kv_splits);
+                                        max_context, kv_splits, seq_lens != nullptr);
     if (plan.bytes > 0 && (!workspace || workspace_bytes < plan.bytes))
         return fail(SFG_ERR_WORKSPACE, "attn_decode_paged: workspace %zu < %zu", workspace_bytes, plan.bytes);
     return launch_paged(plan, q, k_pool, v_pool, SFG_BF16, page_table, seq_lens, out, out_dtype, batch,
@@ -573,7 +575,7 @@ int sfg_hip_attn_decode_paged_noalloc_v1(const float* q, const uint16_t* k_pool,
                                page_tokens, pages_per_seq, num_pages, max_context);
     if (rc != SFG_OK) return rc;
     const DecodePlan plan = plan_decode(SFG_BF16, batch, q_heads, kv_heads, 1, head_dim, page_tokens,
-                                        max_context, kv_splits);
+                                        max_context, kv_splits, seq_lens != nullptr);
     if (plan.bytes > SFG_DECODE_SCRATCH_BYTES)
         return fail(SFG_ERR_WORKSPACE,
                     "attn_decode_paged_noalloc: %zu bytes of split partials (batch %lld x %lld heads x "
@@ -621,7 +623,7 @@ int sfg_hip_attn_paged_v1(const float* q, const void* k_pool, const void* v_pool
                                 stream)) != SFG_OK)
         return rc;
     const DecodePlan plan = plan_decode(kv_dtype, batch, q_heads, kv_heads, seq_q, head_dim, page_tokens,
-                                        max_context, kv_splits);
+                                        max_context, kv_splits, seq_lens != nullptr);
     if (plan.bytes > 0 && (!workspace || workspace_bytes < plan.bytes))
         return fail(SFG_ERR_WORKSPACE, "attn_paged: workspace %zu < %zu", workspace_bytes, plan.bytes);
     return launch_paged(plan, q, k_pool, v_pool, kv_dtype, page_table, seq_lens, out, out_dtype, batch,
@@ -876,7 +878,7 @@ int validate_desc(const sfg_layer_desc* d) {
 DecodePlan layer_decode_plan(const sfg_layer_desc* d) {
     const int64_t keys = static_cast<int64_t>(d->context) + (d->kv_append ? d->sequence : 0);
     return plan_decode(d->act_dtype, d->batch, d->query_heads, d->kv_heads, d->sequence, d->head_dim,
-                       d->page_tokens, keys, d->kv_splits);
+                       d->page_tokens, keys, d->kv_splits, d->kv_append != 0);
 }
 
 // The flash prefill over V^T serves bf16 activations at head_dim 128.

@@ -1021,19 +1021,28 @@ __global__ __launch_bounds__(kDecD) void attn_decode_combine_kernel(
     else out[static_cast<int64_t>(bh) * kDecD + d] = f32_to_bf16(o);
 }
 
-int decode_split_count(int64_t batch, int64_t kv_heads, int64_t max_context, int64_t page_tokens,
-                       int32_t requested) {
+int decode_split_count(int64_t batch, int64_t kv_heads, int64_t head_dim, int64_t max_context, int64_t page_tokens,
+                       int32_t requested, bool ragged) {
     const int64_t pages = (max_context + page_tokens - 1) / page_tokens;
     if (requested > 0) return static_cast<int>(requested < pages ? requested : (pages > 0 ? pages : 1));
+    const int64_t base = batch * kv_heads;
     // Aim for >= 1024 workgroups while keeping >= 32 pages (8 per wave) each.
     int s = 1;
-    while (batch * kv_heads * s < 1024 && pages / (s * 2) >= 32) s *= 2;
+    while (base * s < 1024 && pages / (s * 2) >= 32) s *= 2;
     // Small batches and short contexts leave CUs idle at that: up to 512
     // workgroups (two per CU) down to 8 pages each.  1 sequence x 8 kv heads x
     // 4096 tokens 15.4 -> 11.6 us (16 splits), x 700 15.8 -> 10.9 (4), 8 x 8 x 2000
     // 24.8 -> 13.0 (8).  Past 16 splits the combine costs more than it gives
     // (1 x 8 x 4096 at 32: 17.4).
-    while (s < 16 && batch * kv_heads * s < 512 && pages / (s * 2) >= 8) s *= 2;
+    const int whole = s;
+    while (s < 16 && base * s < 512 && pages / (s * 2) >= 8) s *= 2;
+    // At head_dim 128 a CU holds two workgroups, so the last doubling can leave a
+    // part of them to a second round.  Sequences of one length then take only as
+    // many splits as fit: 6 x 16 heads x 2206 tokens 24.8 us at 8, 21.2 at 5 (22.5 at
+    // the 4 that keep 32 pages each), 24 x 16 x 276 19.1 at 2, 15.4 at 1.  Sequences with
+    // lengths of their own leave early workgroups' places to the second round, and
+    // the finer split evens them out: 34 x 8 x up to 707 16.0 us at 2, 22.2 at 1.
+    if (!ragged && head_dim > 64 && s > whole && base * s > 512) s = static_cast<int>(std::max<int64_t>(whole, 512 / base));
     return s;
 }
 

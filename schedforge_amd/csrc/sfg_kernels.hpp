@@ -103,8 +103,8 @@ int launch_attn_prefill_vt(const uint16_t* q, const uint16_t* k, const uint16_t*
                            int causal, float scale, int waves, hipStream_t stream);
 void launch_v_transpose(const float* qkv, int64_t batch, int64_t seq, int64_t q_heads,
                         int64_t kv_heads, int64_t ld_vt, uint16_t* vt, hipStream_t stream);
-int decode_split_count(int64_t batch, int64_t kv_heads, int64_t max_context,
-                       int64_t page_tokens, int32_t requested);
+int decode_split_count(int64_t batch, int64_t kv_heads, int64_t head_dim, int64_t max_context,
+                       int64_t page_tokens, int32_t requested, bool ragged);
 size_t decode_workspace_bytes(int64_t batch, int64_t q_heads, int64_t head_dim, int splits);
 // The MFMA split-KV decode: bf16 pools, head_dim 64 / 128, 16-token pages, one
 // new token per sequence, GQA group 1 / 2 / 4 / 8 / 16 (decode_mfma_supported);

@@ -216,3 +216,29 @@ def test_automatic_split_counts_match_one_split(b, hkv, longest):
         torch.cuda.synchronize()
         outs.append(host(out))
     np.testing.assert_allclose(outs[0], outs[1], atol=2.0 ** -8 * np.abs(outs[1]).max())
+
+
+# batches whose last doubling of the splits would start a second round of workgroups:
+# without lengths of their own they take as many splits as fit, powers of two or not
+@pytest.mark.parametrize("b,hkv,longest,d", [(6, 16, 2206, 128), (24, 16, 276, 128), (3, 8, 4096, 128), (6, 16, 2206, 64),
+                                             (40, 2, 1500, 128)])
+def test_split_counts_of_equal_sequences_match_one_split(b, hkv, longest, d):
+    lib = _abi.load()
+    rng = np.random.default_rng(longest + b)
+    hq, pps = hkv, (longest + PT - 1) // PT
+    table = rng.permutation(b * pps).reshape(b, pps).astype(np.int32)
+    k, v = (bf16_dev(rng.standard_normal(s).astype(np.float32)) for s in ((b * pps, hkv, PT, d), (b * pps, hkv, d, PT)))
+    q, td, ld = dev(rng.standard_normal((b, hq, 1, d)).astype(np.float32)), dev(table), dev(np.full(b, longest, np.int32))
+    outs = []
+    for splits, lens in ((0, None), (0, ld.data_ptr()), (1, None)):
+        n = lib.sfg_hip_attn_paged_workspace_v1(b, hq, hkv, 1, d, BF16, longest, PT, splits)
+        out = torch.zeros((b, hq, d), device="cuda")
+        ws = torch.full((max(1, n),), 255, dtype=torch.uint8, device="cuda")
+        KEEP_ALIVE.extend([out, ws])
+        _abi.check(lib.sfg_hip_attn_paged_v1(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), BF16, td.data_ptr(), lens, out.data_ptr(), F32, b, hq, hkv,
+            1, d, PT, pps, b * pps, longest, 1, splits, ctypes.c_float(0.0), 0, ws.data_ptr(), ws.numel(), stream()))
+        torch.cuda.synchronize()
+        outs.append(host(out))
+    for got in outs[:2]:
+        np.testing.assert_allclose(got, outs[2], atol=2.0 ** -8 * np.abs(outs[2]).max())
