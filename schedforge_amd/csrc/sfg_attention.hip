@@ -1293,8 +1293,11 @@ __device__ __forceinline__ uint32_t finite_bf16x2(uint32_t w) {
     return w & ~((bad >> 15) * 0xFFFFu);
 }
 
+// (The bounds keep the registers of the second walk out of the way: at head_dim 64
+// three waves per SIMD instead of four cost 10%.)
 template <typename KvT, int kDecD>
-__global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs p, int chunks) {
+__global__ __launch_bounds__(256, sizeof(KvT) == 2 ? (kDecD == 64 ? 4 : 2) : 1)
+void attn_paged_mfma_rows_kernel(PagedRowsArgs p, int chunks) {
     // 16-column blocks per workgroup; two leave one wave per SIMD (27.8 against
     // 23.0 us on the shape above, though each K / V byte is then read once)
     constexpr int NCB = 1;
@@ -1409,7 +1412,8 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
         for (int dt = 0; dt < kDt; ++dt) vb[dt] = *reinterpret_cast<const VecV*>(vpool + base + dt * 16 * kPageTok);
     };
     // the second walk is for bf16 pools with visible non-finite elements
-    for (int walk = 0;; ++walk) {
+    auto walk_pages = [&](auto second_c) __attribute__((always_inline)) {
+        constexpr bool kSecond = decltype(second_c)::value;
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) {
             m_run[cb] = -INFINITY;
@@ -1430,7 +1434,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
             if (pg + 1 < w_end) load_page(pg + 1);
             const int tok0 = pg * kPageTok + 4 * lg;  // this lane's four tokens
             bool slow = false;
-            if (!ok || walk > 0 || (pg + 1) * kPageTok > all_see) {  // wave-uniform
+            if (!ok || kSecond || (pg + 1) * kPageTok > all_see) {  // wave-uniform
                 // tokens past the end (or of no page) are not data
                 bool bad = false;
 #pragma unroll
@@ -1475,19 +1479,15 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
                 } else {
                     // three independent chains, the small terms summed first
                     floatx4 st3[3] = {floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}, floatx4{0.f, 0.f, 0.f, 0.f}};
-                    auto scores = [&](auto finite_c) __attribute__((always_inline)) {
 #pragma unroll
-                        for (int s = 0; s < kKs; ++s)
+                    for (int s = 0; s < kKs; ++s)
 #pragma unroll
-                            for (int t = 0; t < 3; ++t) {
-                                uint4 k = kc[s];
-                                if (decltype(finite_c)::value && t > 0)
-                                    k = make_uint4(finite_bf16x2(k.x), finite_bf16x2(k.y), finite_bf16x2(k.z), finite_bf16x2(k.w));
-                                st3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), qf[cb][s].t[t], st3[t], 0, 0, 0);
-                            }
-                    };
-                    if (walk == 0) scores(std::false_type{});
-                    else scores(std::true_type{});
+                        for (int t = 0; t < 3; ++t) {
+                            uint4 k = kc[s];
+                            if (kSecond && t > 0)
+                                k = make_uint4(finite_bf16x2(k.x), finite_bf16x2(k.y), finite_bf16x2(k.z), finite_bf16x2(k.w));
+                            st3[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(as_bf16x8(k), qf[cb][s].t[t], st3[t], 0, 0, 0);
+                        }
                     st = st3[0] + (st3[1] + st3[2]);
                 }
                 float sv[4];
@@ -1565,7 +1565,9 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
                 }
             }
         }
-        if (kF32 || walk > 0) break;
+    };
+    walk_pages(std::false_type{});
+    if constexpr (!kF32) {
         bool bad = false;
 #pragma unroll
         for (int cb = 0; cb < NCB; ++cb) {
@@ -1576,7 +1578,7 @@ __global__ __launch_bounds__(256) void attn_paged_mfma_rows_kernel(PagedRowsArgs
                 for (int r = 0; r < 4; ++r) t = fmaf(acc[cb][dt][r], 0.f, t);
             bad |= kend[cb] > 0 && t != 0.f;
         }
-        if (!__any(bad)) break;
+        if (__any(bad)) walk_pages(std::true_type{});
     }
     // merge the four waves in LDS: acc[cb][dt][r] = O^T[dim 16 dt + 4 lg + r][column lr]
     constexpr int kCols = 16 * NCB;
