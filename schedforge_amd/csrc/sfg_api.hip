@@ -371,8 +371,13 @@ int sfg_hip_rmsnorm_v1(const float* x, const float* w, void* y, int y_dtype, int
 }
 
 size_t sfg_hip_gemm_workspace_v1(int64_t m, int64_t n, int64_t k) {
-    const size_t plain = sfg::gemm_workspace_bytes(m, n, k), glu = sfg::gemm_workspace_bytes(m, 2 * n, k);
-    return plain > glu ? plain : glu;
+    size_t most = 0;  // over the weight types and epilogues
+    for (const int dt : {SFG_BF16, SFG_I8})
+        for (const bool glu : {false, true}) {
+            const size_t s = sfg::gemm_workspace_bytes(dt, m, n, k, glu);
+            if (s > most) most = s;
+        }
+    return most;
 }
 
 int sfg_hip_gemm_v1(const sfg_gemm_args* a, void* workspace, size_t workspace_bytes, void* stream) {
@@ -924,13 +929,19 @@ LayerBuffers plan_buffers(const sfg_layer_desc* d, void* ws) {
         b.act = c.take(rows * I * ae);
     }
     if (d->context > 0) b.attn_ws = c.take(layer_decode_plan(d).bytes);
-    // Split-K scratch sized for the widest projection.
+    // Split-K scratch sized for the widest dense product (expert products never
+    // split, and the QKV product of a fused prefill does not either).
     size_t g = 0;
-    const int64_t ns[4] = {qkvw, H, 2 * I, H};
-    const int64_t ks[4] = {H, H, H, I};
-    for (int i = 0; i < 4; ++i) {
-        const size_t s = sfg::gemm_workspace_bytes(rows, ns[i], ks[i]);
+    auto split_scratch = [&](int64_t n, int64_t k, bool glu) {
+        const size_t s = sfg::gemm_workspace_bytes(d->weight_dtype, rows, n, k, glu);
         if (s > g) g = s;
+    };
+    const bool fused_qkv = use_vt(d) && d->weight_layout == SFG_LAYOUT_NK && rows > 64 && d->sequence % 4 == 0;
+    if (!fused_qkv) split_scratch(d->context > 0 && !d->kv_append ? H : qkvw, H, false);
+    split_scratch(H, H, false);
+    if (!moe) {
+        split_scratch(I, H, true);
+        split_scratch(H, I, false);
     }
     b.gemm_ws_bytes = g;
     b.gemm_ws = c.take(g);

@@ -452,7 +452,7 @@ struct SplitReduceArgs {
 
 template <int EPI>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(SplitReduceArgs p) {
-    // four consecutive output columns per thread (n is a multiple of 64); the
+    // four consecutive output columns per thread (n is a multiple of 4); the
     // slices' loads are all issued before the ordered sum
     const int64_t idx = (static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x) * 4;
     if (idx >= p.m * p.n) return;
@@ -1814,10 +1814,13 @@ bool mfma_operands(const GemmProblem& p) {
 
 // The tile launch_gemm gives a product on the ring / 256 x 256 kernels.
 // (int8: the QKV epilogue of a 128 x 128 wave block does not fit the registers;
-// the bf16 256 x 256 tile reads [N][K] only.)
-RingPlan tile_plan(const GemmProblem& p, bool glu, int groups, bool split, size_t workspace_bytes) {
-    const bool allow_v = p.b_dtype == SFG_BF16 ? p.b_layout == SFG_LAYOUT_NK : p.epilogue != kEpiQkvRope;
-    return ring_plan(p.b_dtype, p.m, p.n, p.k, glu, groups, split, allow_v, workspace_bytes);
+// gemm_dma_kernel's tiles read [N][K] only.)
+RingPlan tile_plan(const GemmProblem& p, int groups, bool split, size_t workspace_bytes) {
+    const bool nk = p.b_layout == SFG_LAYOUT_NK, qkv = p.epilogue == kEpiQkvRope;
+    RingAsk q{p.b_dtype, p.m, p.n, p.k, p.epilogue, qkv ? SFG_BF16 : p.c_dtype, groups, split, false, false, workspace_bytes};
+    q.allow_v = p.b_dtype == SFG_BF16 ? nk : !qkv;
+    q.allow_dma = p.b_dtype == SFG_BF16 && nk && !qkv;
+    return ring_plan(q);
 }
 
 bool gemm_qkv_rope_supported(const GemmProblem& p) {
@@ -1833,7 +1836,7 @@ bool gemm_qkv_rope_supported(const GemmProblem& p) {
     // than the separate split + RoPE pass costs.
     if (o.seq % 4 == 0) return true;
     const bool named = p.b_dtype == SFG_BF16 && p.m >= kBigMinRows && p.tile > SFG_TILE_AUTO;
-    return !named && tile_plan(p, false, 1, false, 0).tile != kRingTileV;
+    return !named && tile_plan(p, 1, false, 0).tile != kRingTileV;
 }
 
 int gemm_preferred_layout(int64_t rows, int64_t k, bool grouped) {
@@ -1842,19 +1845,13 @@ int gemm_preferred_layout(int64_t rows, int64_t k, bool grouped) {
     return skinny ? SFG_LAYOUT_TILED : SFG_LAYOUT_NK;
 }
 
-size_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k) {
-    if (m <= 0 || n <= 0 || k <= 0) return 0;
-    if (m <= kSkinnyMaxRows) return splitk_bytes(m, n, k);
-    if (m >= kBigMinRows) return 0;  // enough tiles without a split
-    // the largest any weight type or epilogue over these B rows would take
-    size_t most = 0;
-    for (const int dt : {SFG_BF16, SFG_I8})
-        for (const bool glu : {false, true}) {
-            if (glu && n % 2) continue;
-            const RingPlan r = ring_plan(dt, m, glu ? n / 2 : n, k, glu, 1, true, true, kRingNoLimit);
-            if (r.part > most) most = r.part;
-        }
-    return most;
+size_t gemm_workspace_bytes(int b_dtype, int64_t m, int64_t n, int64_t k, bool glu) {
+    const int64_t nb = glu ? 2 * n : n;
+    if (m <= 0 || n <= 0 || k <= 0 || b_dtype == SFG_F32) return 0;  // (fp32 products never split)
+    if (m <= kSkinnyMaxRows) return splitk_bytes(m, nb, k);
+    if (m >= kBigMinRows || gemm_short_k(b_dtype, m, n, k, glu, 1)) return 0;
+    return ring_plan(RingAsk{b_dtype, m, n, k, glu ? SFG_EPI_SWIGLU : SFG_EPI_NONE, SFG_F32, 1, true, true, false,
+                             kRingNoLimit}).part;
 }
 
 int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_bytes,
@@ -1874,8 +1871,10 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
             !fits_32bit(a_rows, p.lda, 4, glu ? 2 * p.n : p.n, p.ldb, 4, 2 * p.k))
             return launch_vec(p, stream);
         const int groups = p.offsets ? p.groups : 1;
-        // one pass over K whatever the rows: no split
-        const RingPlan plan = ring_plan(SFG_F32, p.m, p.n, p.k, glu, groups, false, false, 0);
+        if (groups == 1 && gemm_f32_short_k(p.m, p.n, p.k, glu)) return launch_vec(p, stream);
+        // No split over workgroups.  (gemm_f32_small_kernel's four waves take every
+        // fourth slab each, so the order of an fp32 sum depends on the tile.)
+        const RingPlan plan = tile_plan(p, groups, false, 0);
         return launch_ring(tiled_args(p, groups), plan, SFG_F32, p.epilogue, nullptr, stream);
     }
     if (p.a_dtype != SFG_BF16 || (p.b_dtype != SFG_BF16 && p.b_dtype != SFG_I8))
@@ -1914,15 +1913,9 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
     const int64_t tile_cols = glu ? 16 * nbt / 2 : 16 * nbt;
     const bool tiled_ok = p.b_layout != SFG_LAYOUT_TILED || p.n % 16 == 0;
     if (skinny_rows && p.n % tile_cols != 0 && p.b_layout == SFG_LAYOUT_TILED) return SFG_ERR_UNSUPPORTED;
-    // Grouped products of many rows per group: the ring tiles read each weight
-    // once, the skinny kernel once per 32 rows of a group.  Eight groups, W1|W3
-    // and W2 together, skinny against ring (us): bf16 H2048 I1408, 128 rows 45 /
-    // 47, 200 rows 56 / 49, 512 rows 110 / 62; H4096 I14336, 128 rows 506 / 538,
-    // 200 rows 649 / 546; int8 H4096 I14336, 200 rows 379 / 403, 256 rows 422 /
-    // 399, 512 rows 764 / 577; int8 H2048 I1408, 128 rows 39 / 39, 256 rows 65 / 41.
-    const int64_t ring_rows = p.b_dtype == SFG_I8 ? 28 : 20;  // rows per group
-    const bool ring_grouped = p.offsets && p.m >= ring_rows * groups && tiled_ok && fits_32bit(p.a_rows ? p.a_rows_limit : p.m, p.lda, 2, nb, p.ldb,
-                                                    p.b_dtype == SFG_I8 ? 1 : 2, p.k);
+    const int64_t ring_rows = gemm_ring_rows(p.b_dtype, glu, groups);
+    const bool small32 = fits_32bit(p.a_rows ? p.a_rows_limit : p.m, p.lda, 2, nb, p.ldb, p.b_dtype == SFG_I8 ? 1 : 2, p.k);
+    const bool ring_grouped = p.offsets && p.m >= ring_rows * groups && tiled_ok && small32;
     const bool skinny = skinny_rows && p.n % tile_cols == 0 && !ring_grouped;
     if (skinny) {
         const int mt = rows_hint <= 16 ? 1 : (rows_hint <= 32 ? 2 : 4);
@@ -1958,23 +1951,25 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
     const bool whole_n = p.n % (glu ? 64 : 128) == 0;
     const bool big = p.k % kGK == 0 && p.m >= kBigMinRows;
     const TiledArgs a = tiled_args(p, groups);
-    if (fits_32bit(a.a_rows_limit, p.lda, 2, nb, p.ldb, p.b_dtype == SFG_I8 ? 1 : 2, p.k)) {
+    const bool named = big && p.b_dtype == SFG_BF16 && p.tile > SFG_TILE_AUTO;
+    const bool short_k = !named && p.b_layout == SFG_LAYOUT_NK && p.epilogue != kEpiQkvRope &&
+                         gemm_short_k(p.b_dtype, p.m, p.n, p.k, glu, groups);
+    if (small32 && !short_k) {
         // A plan that names a direct-to-LDS tile gets it (bf16, >= 1024 rows);
-        // otherwise the ring tiles and the 256 x 256 one compete.  From 1024
+        // otherwise the ring tiles and the direct-to-LDS ones compete.  From 1024
         // rows on no product splits K, so every tile gives the same bits.
-        const bool named = big && p.b_dtype == SFG_BF16 && p.tile > SFG_TILE_AUTO;
         // (the reduce reads the partials as 16-byte vectors)
         const bool split = !p.offsets && !p.a_rows && p.epilogue != kEpiQkvRope && p.m < kBigMinRows &&
                            workspace && (reinterpret_cast<uintptr_t>(workspace) & 15) == 0;
         RingPlan plan{};
-        if (!named) plan = tile_plan(p, glu, groups, split, workspace_bytes);
-        if (!named && (plan.tile != kRingTileV || p.b_dtype != SFG_BF16)) {
+        if (!named) plan = tile_plan(p, groups, split, workspace_bytes);
+        if (!named && plan.tile != kRingTileDma && (plan.tile != kRingTileV || p.b_dtype != SFG_BF16)) {
             float* const part = plan.splits > 1 ? static_cast<float*>(workspace) : nullptr;
             const int rc = launch_ring(a, plan, p.b_dtype, p.epilogue, part, stream);
             if (rc == SFG_OK && part) launch_splitk_reduce(p, part, plan.splits, nb, stream);
             return rc;
         }
-        const DmaShape sh = dma_shape_of(named ? p.tile : SFG_TILE_256x256_V);
+        const DmaShape sh = dma_shape_of(named ? p.tile : plan.tile == kRingTileDma ? SFG_TILE_256x128 : SFG_TILE_256x256_V);
         const int64_t cols = glu ? sh.bn / 2 : sh.bn;
         const int64_t tn = (p.n + cols - 1) / cols;
         const int64_t tm = (p.m + sh.bm - 1) / sh.bm;
@@ -1993,7 +1988,7 @@ int launch_gemm(const GemmProblem& problem, void* workspace, size_t workspace_by
         else launch_dma_b<128, 128>(a, grid, itm, static_cast<int>(tn), p.epilogue, stream);
         return SFG_OK;
     }
-    if (big && whole_n) {
+    if (big && whole_n && !short_k) {
         const int64_t tn = glu ? p.n / 64 : p.n / 128;
         if (p.offsets) {
             const dim3 grid(static_cast<unsigned>(tn), static_cast<unsigned>((p.m + kGM - 1) / kGM + groups));

@@ -530,72 +530,6 @@ __global__ __launch_bounds__(256) void gemm_f32_small_kernel(TiledArgs p, int ti
     }
 }
 
-// ===========================================================================
-// Host side: tile and split choice.
-// ===========================================================================
-namespace {
-
-// One tile of the choice: its workgroups per CU and microseconds per 64-k slab
-// with every CU busy (bf16 / int8 weights).  The slab times are what the L2
-// miss path gives one CU: it moves 45 - 55 KB/us whatever the ring depth (four
-// and five stages, and 32 to 256 workgroups, measured within 3%), so a slab
-// costs its bytes, and larger tiles win until they leave CUs idle.
-struct RingTile {
-    int tile, bm, bn, per_cu;
-    float us_bf16, us_i8, us_f32;
-    bool glu;
-};
-constexpr RingTile kRingTiles[] = {
-    {kRingTileV, 256, 256, 1, 1.55f, 1.60f, 0.f, true},
-    {kRingTile256x128, 256, 128, 1, 1.10f, 1.05f, 3.80f, true},
-    {kRingTile128x128, 128, 128, 1, 0.69f, 0.64f, 1.90f, true},
-    {kRingTile64x128, 64, 128, 1, 0.52f, 0.52f, 1.00f, true},
-    {kRingTile128x64, 128, 64, 1, 0.52f, 0.48f, 1.00f, false},
-    {kRingTile64x64, 64, 64, 2, 0.56f, 0.50f, 1.00f, false},
-    {kRingTileSmall, 32, 32, 1, 0.f, 0.f, 0.13f, true},
-};
-constexpr int kRingCus = 256;
-constexpr size_t kRingMaxPart = size_t(64) << 20;  // bytes of split-K partials
-
-}  // namespace
-
-RingPlan ring_plan(int b_dtype, int64_t m, int64_t n, int64_t k, bool glu, int groups, bool may_split,
-                   bool allow_v, size_t workspace) {
-    const int64_t slab_k = b_dtype == SFG_F32 ? 32 : 64;
-    const int64_t slabs = (k + slab_k - 1) / slab_k;
-    const int64_t nb = glu ? 2 * n : n;
-    RingPlan best{};
-    float best_us = 0.f;
-    for (const RingTile& t : kRingTiles) {
-        float us = b_dtype == SFG_I8 ? t.us_i8 : b_dtype == SFG_F32 ? t.us_f32 : t.us_bf16;
-        if (us == 0.f || (glu && !t.glu) || (t.tile == kRingTileV && (!allow_v || (b_dtype == SFG_BF16 && k % 64 != 0))))
-            continue;
-        const bool small = t.tile == kRingTileSmall;  // 32 output columns either way
-        const int64_t cols = glu && !small ? t.bn / 2 : t.bn;
-        if (small && glu) us *= 2.f;
-        // grouped: half a tile of padding per group on average
-        const int64_t rows = (m + t.bm - 1) / t.bm + (groups > 1 ? groups / 2 : 0);
-        const int64_t tiles = rows * ((n + cols - 1) / cols);
-        for (int s = 1; s <= 16; ++s) {
-            const size_t part = s > 1 ? static_cast<size_t>(s) * m * nb * 4 : 0;
-            if (s > 1 && (!may_split || groups > 1 || t.tile == kRingTileV || small || n % 4 != 0 || slabs / s < 4 ||
-                          part > kRingMaxPart || part > workspace))
-                break;
-            const int64_t room = static_cast<int64_t>(kRingCus) * t.per_cu;
-            const float rounds = static_cast<float>((tiles * s + room - 1) / room);
-            // 3 us of prologue and epilogue a round; a split adds its reduce
-            // launch and one write and one read of the partials (4 TB/s)
-            float time = rounds * (static_cast<float>((slabs + s - 1) / s) * us + 3.f);
-            if (s > 1) time += 4.f + static_cast<float>(part) * 2.f / 4.0e6f;
-            if (best_us == 0.f || time < best_us) {
-                best_us = time;
-                best = RingPlan{t.tile, t.bm, t.bn, s, part};
-            }
-        }
-    }
-    return best;
-}
-
 namespace {
 
 template <int BDT, int BM, int BN, int NW, int NS>

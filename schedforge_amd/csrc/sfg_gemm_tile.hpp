@@ -5,6 +5,7 @@
 
 #include <type_traits>
 
+#include "sfg_gemm_plan.hpp"
 #include "sfg_kernels.hpp"
 
 namespace sfg {
@@ -32,26 +33,14 @@ struct TiledArgs {
     void* c; int c_dtype; int64_t ldc;
     const float* residual; int64_t ldr;
     int64_t m, n, k;
-    const int32_t* offsets;   // grouped: tiles per group = ceil(rows_g / 128)
+    const int32_t* offsets;   // grouped: first row of each group
     int groups;
     QkvRopeOut qkv;           // kEpiQkvRope only
     int xcds;                 // XCDs the dispatcher deals workgroups over
     int b_tiled;              // gemm_ring_kernel: B in SFG_LAYOUT_TILED
 };
 
-// The middle-size GEMM (sfg_gemm_ring.hip): tile and K split chosen for a
-// product; with bf16 weights kRingTileV is the 256 x 256 64-k-slab tile of
-// gemm_dma_kernel.  `part` bytes of split-K partial sums ([splits][m][B rows]
-// fp32) come from the caller's workspace.
-enum { kRingTileV = 1, kRingTile256x128, kRingTile128x128, kRingTile64x128, kRingTile128x64, kRingTile64x64,
-       kRingTileSmall /* fp32 only: gemm_f32_small_kernel */ };
-constexpr size_t kRingNoLimit = ~size_t(0);
-struct RingPlan {
-    int tile, bm, bn, splits;
-    size_t part;
-};
-RingPlan ring_plan(int b_dtype, int64_t m, int64_t n, int64_t k, bool glu, int groups, bool may_split,
-                   bool allow_v, size_t workspace);
+// (sfg_gemm_ring.hip)
 int launch_ring(const TiledArgs& a, const RingPlan& plan, int b_dtype, int epi, float* part, hipStream_t s);
 
 // ===========================================================================

@@ -67,7 +67,8 @@ int device_xcds(hipStream_t stream);
 int device_cus(hipStream_t stream);
 
 bool gemm_qkv_rope_supported(const GemmProblem& p);
-size_t gemm_workspace_bytes(int64_t m, int64_t n, int64_t k);
+// Split-K scratch of a dense product of n outputs (2 n B rows for GLU).
+size_t gemm_workspace_bytes(int b_dtype, int64_t m, int64_t n, int64_t k, bool glu);
 // The layout launch_gemm reads fastest for these rows (see sfg_layout).
 int gemm_preferred_layout(int64_t rows, int64_t k, bool grouped);
 // Returns SFG_OK or an error code (unsupported combination).
