@@ -53,83 +53,13 @@ int launch_ring(const TiledArgs& a, const RingPlan& plan, int b_dtype, int epi, 
 // Every 32-column block lies inside one head, so the Q / K / V choice is
 // uniform per block.  A lane's four consecutive rows (r % 4) are four
 // consecutive tokens of one sequence (S % 4 == 0, checked on the host), so
-// V^T takes one 8-byte store per lane and block.
+// V^T takes one 8-byte store per lane and block.  kAnySeq: sequences of any length
+// of at least four rows, where a run of four rows may end one and begin the next,
+// and V^T takes single stores unless S % 4 == 0.  (Wave blocks larger than 64 x 64
+// have no registers for it.)
 // ===========================================================================
-template <int WM, int WN>
+template <int WM, int WN, bool kAnySeq>
 __device__ __forceinline__ void qkv_rope_epilogue(const QkvRopeOut& o, const floatx16 (&acc)[WM][WN],
-                                                  int64_t wave_row0, int64_t wave_col0, int64_t re,
-                                                  int64_t n, int l32, int khalf) {
-    const int64_t H = static_cast<int64_t>(o.q_heads) * 128;
-    const int64_t kvd = static_cast<int64_t>(o.kv_heads) * 128;
-    const int seq = static_cast<int>(o.seq);
-#pragma unroll
-    for (int i = 0; i < WM; ++i) {
-        // One 32-row block: positions and (cos, sin) of all its rows and this
-        // lane's columns are fetched first, so the block waits for the table
-        // once instead of once per element.
-        int bq[4], sq[4];
-#pragma unroll
-        for (int rq = 0; rq < 4; ++rq) {
-            const int rr = static_cast<int>(wave_row0 + i * 32 + 8 * rq + 4 * khalf);
-            bq[rq] = rr / seq;
-            sq[rq] = rr - bq[rq] * seq;
-        }
-        float2 cs[WN][4][4];
-#pragma unroll
-        for (int j = 0; j < WN; ++j) {
-            const int64_t col = wave_col0 + j * 32 + l32;
-            const bool rot = col < H + kvd;  // uniform over the 32-column block
-            const int pr = static_cast<int>(col & 127) >> 1;
-#pragma unroll
-            for (int rq = 0; rq < 4; ++rq)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    cs[j][rq][e] = rot ? o.rope[static_cast<int64_t>(sq[rq] + e) * 64 + pr] : make_float2(1.f, 0.f);
-        }
-#pragma unroll
-        for (int rq = 0; rq < 4; ++rq) {
-            const int64_t row = wave_row0 + i * 32 + 8 * rq + 4 * khalf;  // rows row .. row + 3
-            const int b = bq[rq], s0 = sq[rq];
-#pragma unroll
-            for (int j = 0; j < WN; ++j) {
-                const int64_t col = wave_col0 + j * 32 + l32;
-                float v[4], pv[4];
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    v[e] = acc[i][j][4 * rq + e];
-                    pv[e] = __shfl_xor(v[e], 1, 64);
-                }
-                if (col >= n || row >= re) continue;
-                const int d = static_cast<int>(col & 127);
-                if (col < H + kvd) {
-                    uint16_t* dst = col < H
-                        ? o.q + ((static_cast<int64_t>(b) * o.q_heads + (col >> 7)) * seq + s0) * 128 + d
-                        : o.k + ((static_cast<int64_t>(b) * o.kv_heads + ((col - H) >> 7)) * seq + s0) * 128 + d;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float2 c = cs[j][rq][e];
-                        // (even, odd) -> (even c - odd s, odd c + even s), the same
-                        // fused operations as qkv_rope_epilogue_staged
-                        const float r0 = (d & 1) ? fmaf(v[e], c.x, pv[e] * c.y) : fmaf(v[e], c.x, -(pv[e] * c.y));
-                        dst[e * 128] = f32_to_bf16(r0);
-                    }
-                } else {
-                    const int64_t hv = (col - H - kvd) >> 7;
-                    uint2 pk;
-                    pk.x = pack_bf16x2(v[0], v[1]);
-                    pk.y = pack_bf16x2(v[2], v[3]);
-                    *reinterpret_cast<uint2*>(o.vt + ((static_cast<int64_t>(b) * o.kv_heads + hv) * 128 + d) * o.ld_vt + s0) = pk;
-                }
-            }
-        }
-    }
-}
-
-// The same for sequences of any length of at least four rows: a run of four rows
-// may end one and begin the next, and V^T takes single stores unless S % 4 == 0.
-// (Larger wave blocks than 64 x 64 have no registers for it.)
-template <int WM, int WN>
-__device__ __forceinline__ void qkv_rope_epilogue_any(const QkvRopeOut& o, const floatx16 (&acc)[WM][WN],
                                                   int64_t wave_row0, int64_t wave_col0, int64_t re,
                                                   int64_t n, int l32, int khalf) {
     const int64_t H = static_cast<int64_t>(o.q_heads) * 128;
@@ -150,7 +80,7 @@ __device__ __forceinline__ void qkv_rope_epilogue_any(const QkvRopeOut& o, const
         // row e of a run of four: its (sequence, position), the run's own unless
         // a sequence ends inside it (sequences hold at least four rows)
         auto row_pos = [&](int rq, int e, int& b, int& sp) __attribute__((always_inline)) {
-            const bool wrap = sq[rq] + e >= seq;
+            const bool wrap = kAnySeq && sq[rq] + e >= seq;
             b = bq[rq] + (wrap ? 1 : 0);
             sp = sq[rq] + e - (wrap ? seq : 0);
         };
@@ -190,7 +120,7 @@ __device__ __forceinline__ void qkv_rope_epilogue_any(const QkvRopeOut& o, const
                     const int64_t head = isq ? col >> 7 : (col - H) >> 7;
 #pragma unroll
                     for (int e = 0; e < 4; ++e) {
-                        if (row + e >= re) break;
+                        if (kAnySeq && row + e >= re) break;
                         int b, sp;
                         row_pos(rq, e, b, sp);
                         const float2 c = cs[j][rq][e];
@@ -201,7 +131,7 @@ __device__ __forceinline__ void qkv_rope_epilogue_any(const QkvRopeOut& o, const
                     }
                 } else {
                     const int64_t hv = (col - H - kvd) >> 7;
-                    if (seq % 4 == 0) {  // four positions of one sequence, 8-byte aligned
+                    if (!kAnySeq || seq % 4 == 0) {  // four positions of one sequence, 8-byte aligned
                         uint2 pk;
                         pk.x = pack_bf16x2(v[0], v[1]);
                         pk.y = pack_bf16x2(v[2], v[3]);
@@ -209,7 +139,7 @@ __device__ __forceinline__ void qkv_rope_epilogue_any(const QkvRopeOut& o, const
                     } else {
 #pragma unroll
                         for (int e = 0; e < 4; ++e) {
-                            if (row + e >= re) break;
+                            if (kAnySeq && row + e >= re) break;
                             int b, sp;
                             row_pos(rq, e, b, sp);
                             o.vt[((static_cast<int64_t>(b) * o.kv_heads + hv) * 128 + d) * o.ld_vt + sp] = f32_to_bf16(v[e]);
@@ -243,8 +173,7 @@ __device__ __forceinline__ void qkv_rope_epilogue_staged(const QkvRopeOut& o, co
     const int64_t kvd = static_cast<int64_t>(o.kv_heads) * 128;
     const int64_t seq = o.seq;
     if (wave_col0 + kCols > n || (wave_col0 >= H + kvd && seq % 8 != 0)) {
-        if constexpr (kAnySeq) qkv_rope_epilogue_any<WM, WN>(o, acc, wave_row0, wave_col0, re, n, l32, khalf);
-        else qkv_rope_epilogue<WM, WN>(o, acc, wave_row0, wave_col0, re, n, l32, khalf);
+        qkv_rope_epilogue<WM, WN, kAnySeq>(o, acc, wave_row0, wave_col0, re, n, l32, khalf);
         return;
     }
     const int col_in_head = static_cast<int>(wave_col0 & 127);  // 0, or 64 for 64-column blocks
@@ -672,8 +601,7 @@ __device__ __forceinline__ void dma_tile_epilogue(const TiledArgs& p, const floa
                                              re, p.n, elane, qkv_stage);
         } else {
             const int64_t wrow0 = row0 + wm * (BM / kWavesM), wcol0 = ncol0 + wn * (BN / kWavesN);
-            if constexpr (kAnySeq) qkv_rope_epilogue_any<WM, WN>(p.qkv, acc, wrow0, wcol0, re, p.n, el32, ekhalf);
-            else qkv_rope_epilogue<WM, WN>(p.qkv, acc, wrow0, wcol0, re, p.n, el32, ekhalf);
+            qkv_rope_epilogue<WM, WN, kAnySeq>(p.qkv, acc, wrow0, wcol0, re, p.n, el32, ekhalf);
         }
     }
 }
