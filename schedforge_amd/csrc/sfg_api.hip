@@ -1017,10 +1017,9 @@ int sfg_hip_decoder_layer_v1(const sfg_layer_desc* d, const sfg_layer_weights* w
     if (rc != SFG_OK) return rc;
     if (!w || !io || !io->x || !io->out) return fail(SFG_ERR_SHAPE, "decoder layer: null weights or io");
     const hipStream_t s = as_stream(stream_ptr);
-    const LayerBuffers need = plan_buffers(d, nullptr);
-    if (!workspace || workspace_bytes < need.total)
-        return fail(SFG_ERR_WORKSPACE, "decoder layer: workspace %zu < %zu", workspace_bytes, need.total);
     const LayerBuffers b = plan_buffers(d, workspace);
+    if (!workspace || workspace_bytes < b.total)
+        return fail(SFG_ERR_WORKSPACE, "decoder layer: workspace %zu < %zu", workspace_bytes, b.total);
     const bool moe = d->ffn == 1;
     const bool decode = d->context > 0;
     const int64_t rows = static_cast<int64_t>(d->batch) * d->sequence;
