@@ -10,6 +10,7 @@
 // an MI355X (GpuCostModel), where the reference sums CPU penalties.
 #include "sfg_decoder.hpp"
 #include "sfg_runtime_internal.hpp"
+#include "../csrc/sfg_gemm_plan.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -22,14 +23,16 @@
 namespace schedforge::hip {
 namespace {
 
+using namespace sfg;
+
 std::int64_t ceil_div(std::int64_t a, std::int64_t b) { return (a + b - 1) / b; }
 
-// The GEMM family's choice, simplified for the estimate: skinny GEMV for few
-// rows, the direct-to-LDS MFMA kernel for bf16 weights and >= 1024 rows, one
-// 128 x 128 tile rate in between, fp32.
+// The GEMM family's choice: skinny GEMV for few rows, the direct-to-LDS kernel's
+// tile where a plan names one (bf16 weights, >= 1024 rows), else the tile and time
+// of the launcher's own estimate (ring_plan).
 constexpr std::int64_t kSkinnyMaxRows = 64;
 constexpr std::int64_t kSkinnyGroupedMaxTotal = 512;
-constexpr std::int64_t kBigMinRows = 1024;
+constexpr std::int64_t kBigMinRows = kRingBigMinRows;
 
 struct TileShape {
     int bm, bn, per_cu;
@@ -47,30 +50,27 @@ TileShape tile_shape(int tile) {
     }
 }
 
-// SFG_TILE_AUTO for the estimate: the largest tile with >= 512 workgroups
-// (256 x 256 on the 64-k slab loop), and that tile for grouped products from
-// 128 workgroups up.  (The launcher also weighs the ring tiles.)
-int auto_tile(std::int64_t m, std::int64_t n_out, bool glu, int groups) {
-    if (groups > 1 && (ceil_div(m, 256) + groups) * ceil_div(n_out, glu ? 128 : 256) >= 128)
-        return SFG_TILE_256x256_V;
-    for (const int t : {SFG_TILE_256x256_V, SFG_TILE_256x128, SFG_TILE_128x128}) {
-        const TileShape s = tile_shape(t);
-        const std::int64_t cols = glu ? s.bn / 2 : s.bn;
-        const std::int64_t tiles = (ceil_div(m, s.bm) + (groups > 1 ? groups : 0)) * ceil_div(n_out, cols);
-        if (tiles >= 512) return t;
-    }
-    return SFG_TILE_128x128;
-}
-
-// The split-KV count the decode launcher picks when the policy leaves it open
-// (decode_split_count in the HIP library): double while the grid stays under
-// 1024 workgroups and each split keeps at least 32 pages, then under 512
-// workgroups and 16 splits while each keeps 8.
+// The split-KV count the decode launcher picks when the policy leaves it open.
+// One bf16 row per sequence (decode_split_count in the HIP library): double while the
+// grid stays under 1024 workgroups and each split keeps at least 32 pages, then under
+// 512 workgroups and 16 splits while each keeps 8; at head_dim 128 no further than
+// 512 workgroups hold.  Several rows or fp32 pools (paged_mfma_rows_split_count): double
+// under 512 workgroups of 16 rows while each split keeps 8 pages.
 int auto_kv_splits(const DecoderConfig& c) {
     const std::int64_t pages = ceil_div(c.context_sequence, c.page_tokens);
     int s = 1;
-    while (static_cast<std::int64_t>(c.batch) * c.kv_heads * s < 1024 && pages / (s * 2) >= 32) s *= 2;
-    while (s < 16 && static_cast<std::int64_t>(c.batch) * c.kv_heads * s < 512 && pages / (s * 2) >= 8) s *= 2;
+    if (c.sequence > 1 || c.precision == DecoderPrecision::F32) {
+        const std::int64_t rows = static_cast<std::int64_t>(c.sequence) * (c.query_heads / c.kv_heads);
+        const std::int64_t groups = static_cast<std::int64_t>(c.batch) * c.kv_heads * ceil_div(rows, 16);
+        while (groups * s < 512 && pages / (s * 2) >= 8) s *= 2;
+        return s;
+    }
+    const std::int64_t base = static_cast<std::int64_t>(c.batch) * c.kv_heads;
+    while (base * s < 1024 && pages / (s * 2) >= 32) s *= 2;
+    const int whole = s;
+    while (s < 16 && base * s < 512 && pages / (s * 2) >= 8) s *= 2;
+    if (c.head_dim > 64 && s > whole && base * s > 512)
+        s = static_cast<int>(std::max<std::int64_t>(whole, 512 / base));
     return s;
 }
 
@@ -96,22 +96,27 @@ struct Terms {
     }
 
     // One product: m rows, n_out outputs (2 n_out weight rows for GLU), k.
-    double gemm_us(std::int64_t mrows, std::int64_t n_out, std::int64_t k, bool glu, int groups) const {
+    double gemm_us(std::int64_t mrows, std::int64_t n_out, std::int64_t k, int epi, int c_dtype, int groups) const {
+        const bool glu = ring_is_glu(epi);
         const std::int64_t n = glu ? 2 * n_out : n_out;
         const double flops = 2.0 * static_cast<double>(mrows) * n * k;
-        if (f32) return flops / (m.valu_fp32_flops * m.fp32_gemm_efficiency) * 1e6 + m.launch_microseconds;
+        const int b_dtype = f32 ? SFG_F32 : (c.precision == DecoderPrecision::W8 ? SFG_I8 : SFG_BF16);
         const bool grouped = groups > 1;
-        const bool skinny = k % 128 == 0 && (grouped ? mrows <= kSkinnyGroupedMaxTotal : mrows <= kSkinnyMaxRows);
+        // the VALU kernel: depths that are not whole 16-byte chunks
+        if (k % (f32 ? 4 : 32) != 0)
+            return flops / (m.valu_fp32_flops * m.fp32_gemm_efficiency) * 1e6 + m.launch_microseconds;
+        const bool skinny = !f32 && k % 128 == 0 && (grouped ? mrows <= kSkinnyGroupedMaxTotal : mrows <= kSkinnyMaxRows) &&
+                            !(grouped && mrows >= gemm_ring_rows(b_dtype, glu, groups) * groups);
         if (skinny) {
             const double eff = q.weight_layout == SFG_LAYOUT_TILED ? m.gemv_tiled_efficiency : m.gemv_nk_efficiency;
             // every group's weights stream once per pass of 32 (grouped) or all rows
             const double passes = grouped ? 1.0 : std::max(1.0, std::ceil(static_cast<double>(mrows) / 64.0));
             return hbm_us(static_cast<double>(groups) * n * k * wbytes * passes, eff) + m.launch_microseconds;
         }
-        const bool big = k % 32 == 0 && mrows >= kBigMinRows && c.precision == DecoderPrecision::BF16;
-        if (big) {
-            const int tile = q.gemm_tile != SFG_TILE_AUTO ? q.gemm_tile : auto_tile(mrows, n_out, glu, groups);
-            const TileShape s = tile_shape(tile);
+        const bool named = q.gemm_tile != SFG_TILE_AUTO && k % 64 == 0 && mrows >= kBigMinRows &&
+                           c.precision == DecoderPrecision::BF16;
+        if (named) {
+            const TileShape s = tile_shape(q.gemm_tile);
             const std::int64_t cols = glu ? s.bn / 2 : s.bn;
             // grouped rows are assumed spread evenly over the groups
             const std::int64_t row_tiles = grouped ? groups * ceil_div(ceil_div(mrows, groups), s.bm)
@@ -121,17 +126,19 @@ struct Terms {
             const double waves = static_cast<double>(ceil_div(tiles, slots));
             const double per_cu = m.mfma_bf16_flops / m.compute_units;
             const double tile_flops = 2.0 * s.bm * s.bn * static_cast<double>(k);
-            const double tile_us = tile_flops * s.per_cu / (per_cu * m.tile_efficiency[tile]) * 1e6;
+            const double tile_us = tile_flops * s.per_cu / (per_cu * m.tile_efficiency[q.gemm_tile]) * 1e6;
             return waves * tile_us + m.launch_microseconds;
         }
-        return flops / (m.mfma_bf16_flops * 0.25) * 1e6 + m.launch_microseconds;
+        RingAsk ask{b_dtype, mrows, n_out, k, epi, c_dtype, groups, !grouped && !f32, !f32, b_dtype == SFG_BF16 && !grouped,
+                    kRingNoLimit};
+        return ring_plan(ask).us * kRingCus / m.compute_units;  // its launch included
     }
 
     double decode_attention_us() const {
         const std::int64_t pages = ceil_div(c.context_sequence, c.page_tokens);
         int splits = q.kv_splits > 0 ? q.kv_splits : auto_kv_splits(c);
         splits = static_cast<int>(std::min<std::int64_t>(splits, std::max<std::int64_t>(1, pages)));
-        const double kv = 2.0 * c.batch * kvd * c.context_sequence * 2.0;
+        const double kv = 2.0 * c.batch * kvd * c.context_sequence * (f32 ? 4.0 : 2.0);
         const double groups = static_cast<double>(c.batch) * c.kv_heads * splits;
         // below two workgroups per CU the stream cannot cover HBM latency
         const double fill = std::min(1.0, groups / (2.0 * m.compute_units));
@@ -146,7 +153,9 @@ struct Terms {
         const double S = c.sequence;
         const double pairs = c.causal ? S * (S + 1.0) / 2.0 : S * S;
         const double flops = 2.0 * (2.0 * D) * pairs * c.batch * c.query_heads;
-        if (f32) return flops / (m.valu_fp32_flops * 0.2) * 1e6 + m.launch_microseconds;
+        // fp32: the flash kernel on the fp32 matrix instructions, or (other head dims)
+        // one wave per query row
+        if (f32) return flops / (m.valu_fp32_flops * (D == 64 || D == 128 ? 0.4 : 0.014)) * 1e6 + m.launch_microseconds;
         if (D != 128) return flops / (m.mfma_bf16_flops * 0.15) * 1e6 + m.launch_microseconds;
         // policy 0 resolves as the library does: 8 once 256-row blocks give
         // at least four workgroups per CU
@@ -168,7 +177,7 @@ struct Terms {
         double us = 0.0;
         // norms (two, plus the fp32 copy the MoE router reads)
         us += 2.0 * (hbm_us(rows * H * (4.0 + act), m.hbm_efficiency) + m.launch_microseconds);
-        us += gemm_us(rows, H + 2 * kvd, H, false, 1);
+        us += gemm_us(rows, H + 2 * kvd, H, SFG_EPI_NONE, decode || f32 || D != 128 ? SFG_F32 : SFG_BF16, 1);
         if (decode) {
             us += decode_attention_us();
         } else {
@@ -176,15 +185,15 @@ struct Terms {
                                        m.launch_microseconds;
             us += prefill_attention_us();
         }
-        us += gemm_us(rows, H, H, false, 1);
+        us += gemm_us(rows, H, H, SFG_EPI_RESIDUAL, SFG_F32, 1);
         if (!moe) {
-            us += gemm_us(rows, I, H, true, 1);
-            us += gemm_us(rows, H, I, false, 1);
+            us += gemm_us(rows, I, H, SFG_EPI_SWIGLU, f32 ? SFG_F32 : SFG_BF16, 1);
+            us += gemm_us(rows, H, I, SFG_EPI_RESIDUAL, SFG_F32, 1);
         } else {
             us += hbm_us(rows * H * 4.0, m.hbm_efficiency) + H * 4.0 / 2.4e3 + m.launch_microseconds;  // router
             us += 5.0 + rows * K * 0.002;                                                             // dispatch
-            us += gemm_us(rows * K, I, H, true, static_cast<int>(E));
-            us += gemm_us(rows * K, H, I, false, static_cast<int>(E));
+            us += gemm_us(rows * K, I, H, SFG_EPI_GLU_SILU_UP, f32 ? SFG_F32 : SFG_BF16, static_cast<int>(E));
+            us += gemm_us(rows * K, H, I, SFG_EPI_NONE, SFG_F32, static_cast<int>(E));
             us += hbm_us(rows * K * H * 4.0 + rows * H * 8.0, m.hbm_efficiency) + m.launch_microseconds;
         }
         return us;

@@ -169,6 +169,20 @@ def test_bench_compile_only_profiles_and_schema(tmp_path):
         assert pre == sorted(pre) and dec == sorted(dec), scale
 
 
+def test_estimates_follow_the_kernels_that_run(tmp_path):
+    """The analytical layer time prices the kernel that each product and attention
+    takes: within 1.5 x of the measured layers (us)."""
+    measured = {"f32": {"medium-prefill-s2048": 533.0, "tiny-prefill-s128": 47.0},
+                "bf16": {"large-prefill-s512": 251.0}}
+    for precision, want in measured.items():
+        out = tmp_path / f"{precision}.csv"
+        r = run_bench(["--compile-only", f"--output={out}", f"--precision={precision}"])
+        assert r.returncode == 0, r.stderr
+        est = {row["profile"]: float(row["analytical_us"]) for row in read_csv(out)}
+        for name, us in want.items():
+            assert us / 1.5 < est[name] < us * 1.5, (precision, name, est[name], us)
+
+
 def test_bench_baseline_suite_compile_only(tmp_path):
     out = tmp_path / "b.csv"
     r = run_bench(["--suite=baseline", "--compile-only", f"--output={out}"])
