@@ -72,8 +72,8 @@ enum sfg_layout { SFG_LAYOUT_NK = 0, SFG_LAYOUT_TILED = 1 };
  * paths (skinny decode GEMV, fp32, int8 and small-M kernels).  The plan
  * optimiser (ExecutablePlanOptimizer, decoder_compiler.cpp:750-861) searches it. */
 enum sfg_gemm_tile {
-    SFG_TILE_AUTO = 0,       /* the fastest by estimate: 256 x 256 as V, or a smaller
-                                tile where that leaves compute units idle          */
+    SFG_TILE_AUTO = 0,       /* the fastest by estimate: 256 x 256 as V, 256 x 128, or
+                                a smaller tile where those leave compute units idle */
     SFG_TILE_256x256_PP = 1, /* eight waves as two ping-pong groups of four          */
     SFG_TILE_256x256_W8 = 2, /* eight waves (2 x 4), 128 x 64 per wave               */
     SFG_TILE_256x256_W4 = 3, /* four waves (2 x 2), 128 x 128 per wave               */
@@ -175,8 +175,9 @@ int sfg_hip_rmsnorm_v1(const float* x, const float* w, void* y, int y_dtype, int
  * and for 65..1023 dense rows whose tiles alone leave compute units idle (at
  * most 64 MiB).  With a smaller workspace (or NULL) the same products run with
  * fewer splits or in a single pass.
- * b_layout SFG_LAYOUT_TILED is read by the decode kernels only: bf16 / int8 B,
- * at most 64 rows (grouped: 512 in all), K % 128 == 0 and N % 16 == 0;
+ * b_layout SFG_LAYOUT_TILED is read by the decode kernels (and the grouped form's
+ * tiles) only: bf16 / int8 B, at most 64 rows (grouped: 512 in all), K % 128 == 0 and
+ * N % 16 == 0;
  * other shapes with tiled B return SFG_ERR_UNSUPPORTED. */
 typedef struct {
     const void* a; int32_t a_dtype; int64_t lda;

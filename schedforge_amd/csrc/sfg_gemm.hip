@@ -18,12 +18,13 @@
 //  * gemm_ring_kernel     (sfg_gemm_ring.hip) 65 rows up, bf16 or int8
 //    weights, dense or grouped: 256x128 .. 64x64 tiles through a deep LDS ring,
 //    split over K under 1024 rows when the caller's workspace holds the sums.
-//  * gemm_dma_kernel      bf16 products large enough for its 256x256 tile
-//    (64-k slabs), and any tile a plan names from 1024 rows on: operands global
+//  * gemm_dma_kernel      bf16 products that its 256x256 tile (64-k slabs) or its
+//    256x128 one takes fastest, and any tile a plan names from 1024 rows on: operands global
 //    -> LDS by DMA, v_mfma_f32_32x32x16_bf16, optional A-row gather and
 //    per-group (expert) segments read from device offsets.
 //  * gemm_mfma256_kernel, gemm_mfma_kernel  operands of 4 GiB and more, which
-//    the 32-bit offsets of the two above do not reach: 256x128 and 128x128
+//    the 32-bit offsets of the two above do not reach (the second also products of
+//    few k slabs, gemm_short_k): 256x128 and 128x128
 //    tiles through padded LDS with register prefetch and 64-bit addresses.
 //  * fp32 operands: gemm_ring_kernel's and gemm_f32_small_kernel's fp32 MFMA
 //    forms (sfg_gemm_ring.hip).

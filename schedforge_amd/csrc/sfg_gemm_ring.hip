@@ -1,17 +1,18 @@
-// sfg_gemm_ring.hip -- the MFMA GEMM of the middle sizes (65 rows up): bf16 or
-// int8 weights, dense or grouped, optionally split over K; and the fp32 GEMM.
+// sfg_gemm_ring.hip -- the MFMA GEMM from 65 rows up: bf16 or int8 weights, dense
+// or grouped, optionally split over K; and the fp32 GEMM.
 #include "sfg_gemm_tile.hpp"
 
 namespace sfg {
 
 // ===========================================================================
-// Ring GEMM: BM x BN output tile, four waves in a 2 x 2 grid, K in slabs of 64
-// through a ring of NS LDS stages filled by DMA (global -> LDS, no registers).
+// Ring GEMM: BM x BN output tile, NW waves (four or eight) two abreast, K in slabs
+// of 64 through a ring of NS LDS stages filled by DMA (global -> LDS, no registers).
 //
 // With 65 .. ~1000 rows a launch has one or two tiles per CU, so nothing else
 // on the CU hides a slab's latency: what bounds the tile is how many bytes it
 // keeps in flight.  The ring holds most of the CU's 160 KB for one workgroup
-// (NS - 1 slabs of 16 - 32 KB in flight), one barrier per 64 k.
+// (NS - 1 slabs of 12 - 48 KB in flight), one barrier per 64 k.  (int8: the
+// conversion bounds it; a slab of half the bytes takes as long.)
 //
 // B rows come from [N][K] or from the fragment-tiled layout (the DMA lanes pick
 // their chunks).  A rows are 128 B with 16-byte chunk c of row r in slot c ^ ((r >> 1) & 7);
