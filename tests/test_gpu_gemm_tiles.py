@@ -102,6 +102,28 @@ def test_tile_is_exact(estimate, kind, tile, m, n, epi, k):
     _check(out, F32, ref.astype(np.float32), glu, f"{kind} {m}x{n}x{k} epi {epi}")
 
 
+# the 256 x 256 tile's bf16 stores: GLU rows through the stages that held the last
+# slab (odd widths: rows that start off 16 bytes), residual in pairs of half blocks
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind,m,n,epi,k", [("i8", 300, 8423, EPI_SWIGLU, 64), ("i8", 300, 8424, EPI_GLU_SILU_UP, 416),
+                                            ("i8", 861, 8257, EPI_RESIDUAL, 96), ("bf16", 1300, 3613, EPI_SWIGLU, 704)])
+def test_256x256_bf16_stores(estimate, kind, m, n, epi, k):
+    assert estimate(DT[kind], m, n, k, epi, BF16, 1) == V
+    lib = _abi.load()
+    rng = np.random.default_rng(m + 5 * n + k)
+    a = rng.integers(-3, 4, size=(m, k)).astype(np.float32)
+    res = rng.integers(-5, 6, size=(m, n)).astype(np.float32)
+    glu = epi != EPI_RESIDUAL
+    bd, b_dtype, sd, bm = _weights(rng, kind, (2 * n if glu else n,), k, 0)
+    ref = _epilogue((torch.from_numpy(a).cuda().double() @ torch.from_numpy(bm).cuda().double().T).cpu().numpy(), epi, n, res)
+    out = torch.full((m, n), 77, dtype=torch.int16, device="cuda")
+    KEEP_ALIVE.append(out)
+    args = _args(bf16_dev(a), BF16, bd, b_dtype, sd, out, BF16, dev(res) if not glu else None, m, n, k, epi, 0, 0)
+    _abi.check(lib.sfg_hip_gemm_v1(ctypes.byref(args), None, 0, stream()))
+    torch.cuda.synchronize()
+    _check(out, BF16, ref.astype(np.float32), glu, f"{kind} {m}x{n}x{k} epi {epi}")
+
+
 # int8 experts whose products take the 256 x 256 tile
 @pytest.mark.gpu
 @pytest.mark.parametrize("epi", [EPI_NONE, EPI_GLU_SILU_UP])
